@@ -34,6 +34,8 @@ void adj_fuse_tiles(const KArgs &a, const std::vector<int> &e_first, const std::
                     const int sb[6], std::vector<int> &quiet, std::vector<int> &noisy);
 hipError_t launch_pair_half_step(bool efield, int storage, int mode, const KArgs &a, int m, hipStream_t s,
                                  bool gen_cells);
+hipError_t launch_step(int em, int hm, const KArgs &a, int m, hipStream_t s);
+int fused_rows();
 int tile_rows();
 int tile_cols();
 int pair_tile_cols();
@@ -73,7 +75,13 @@ struct fdtd_ctx {
     bool pair_gen_cells = false;    // ... except the general variant, which runs one cell per thread
     int pair_tiles_x = 0, pair_kchunk = 0;
     int kchunk_h = 0;               // planes per block of the one-cell H sweep (E: ka.kchunk)
-    int box[2][6] = {};             // interior tile box per sweep (0 = E, 1 = H)
+    int box[3][6] = {};             // interior tile box per sweep (0 = E, 1 = H, 2 = the fused step)
+    // fused step: the other buffer of each field and of each psi of the E
+    // sweep, swapped with the current one after a step
+    bool fused = false;
+    int kchunk_f = 0;               // planes per block
+    void *fields2[6] = {};
+    void *psi2[12] = {};            // (psi_h: null, updated in place)
     double step_ms = 0.0;
     size_t psi_elems[12] = {};
     uint64_t dev_bytes = 0;
@@ -192,6 +200,8 @@ void free_device(fdtd_ctx *c)
     for (auto &p : c->psi) p = nullptr;
     for (auto &q : c->qexp) q = nullptr;
     for (auto &q : c->qarr) q = nullptr;
+    for (auto &f : c->fields2) f = nullptr;
+    for (auto &p : c->psi2) p = nullptr;
 }
 
 // The buffers holding the current state.
@@ -209,6 +219,11 @@ int zero_state(fdtd_ctx *c)
     for (int f = 0; f < 6; ++f) {
         if (c->fields[f]) HIPCHK(c, hipMemsetAsync(c->fields[f], 0, (size_t)c->field_elems * c->esz, c->stream));
     }
+    for (int f = 0; f < 6; ++f)
+        if (c->fields2[f]) HIPCHK(c, hipMemsetAsync(c->fields2[f], 0, (size_t)c->field_elems * c->esz, c->stream));
+    for (int p = 0; p < 12; ++p)
+        if (c->psi_elems[p] && c->psi2[p])
+            HIPCHK(c, hipMemsetAsync(c->psi2[p], 0, c->psi_elems[p] * c->esz, c->stream));
     for (int q = 0; q < 2; ++q)
         if (c->qarr[q]) HIPCHK(c, hipMemsetAsync(c->qarr[q], 0, c->qarr_bytes, c->stream));
     for (int p = 0; p < 12; ++p)
@@ -233,7 +248,7 @@ int upload_tables(fdtd_ctx *c);
 // three with a number of blocks along z; FDTD_E_PLANES, FDTD_H_PLANES and
 // FDTD_PAIR_PLANES set one sweep's planes per block before the small-grid
 // halving).
-int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_env)
+int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_env, long min_wg = 1024)
 {
     const char *ov = std::getenv("FDTD_CHUNKS");
     if (const char *pe = std::getenv(planes_env)) planes = std::max(1, std::atoi(pe));
@@ -241,8 +256,7 @@ int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_e
     // workgroups (4 per CU), down to one plane (FDTD_MIN_WG overrides 1024).
     // Measured: 64^3 FP32 18.4 -> 22.7 G, FP16 10.3 -> 22.3 G; 128x128x64
     // FP32 keeps its 4-plane E blocks (2-plane ones measured 3.5 % slower).
-    const char *mw = std::getenv("FDTD_MIN_WG");
-    const long min_wg = mw ? std::atol(mw) : 1024;
+    if (const char *mw = std::getenv("FDTD_MIN_WG")) min_wg = std::atol(mw);
     while (planes > 1 && (long)tiles * (c->in.nz / planes) < min_wg) planes /= 2;
     int nchunks = ov ? std::atoi(ov)
                      : std::min((32 * 1024 * 8 / planes + tiles - 1) / tiles, c->in.nz / planes);
@@ -262,7 +276,9 @@ int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_e
 // z-blocks beside a general one measured slower than the general variant
 // alone: 32.4 against 26.9 ms for 1000 steps; the two half-size launches
 // of a small grid leave CUs idle.)
-void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int kchunk)
+// beyond: cells past the tile's high sides that must lie off the slabs too
+// (the fused step evaluates one).
+void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int beyond = 0)
 {
     const SceneIn &in = c->in;
     const int *L = in.cpml.thick;
@@ -270,7 +286,6 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int kchunk)
     for (int q = 0; q < 6; ++q) ib[q] = 0;
     const char *ev = std::getenv("FDTD_INTERIOR");
     if (ev && std::strcmp(ev, "0") == 0) return;
-    const int by = tile_rows();
     const int nts[3] = {(in.nx + tile_cols - 1) / tile_cols, (in.ny + by - 1) / by, (in.nz + kchunk - 1) / kchunk};
     const int w[3] = {tile_cols, by, kchunk}, nn[3] = {in.nx, in.ny, in.nz};
     int box[6];
@@ -278,7 +293,7 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int kchunk)
         const int lo_cells = std::max(L[2 * ax], 1), hi_cells = nn[ax] - std::max(L[2 * ax + 1], 1);
         int lo = nts[ax], hi = 0;
         for (int t = 0; t < nts[ax]; ++t)
-            if (t * w[ax] >= lo_cells && (t + 1) * w[ax] <= hi_cells) {
+            if (t * w[ax] >= lo_cells && (t + 1) * w[ax] + beyond <= hi_cells) {
                 lo = std::min(lo, t);
                 hi = t + 1;
             }
@@ -287,6 +302,55 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int kchunk)
         box[ax + 3] = hi;
     }
     for (int q = 0; q < 6; ++q) ib[q] = box[q];
+}
+
+// The fused step's tiling and its second buffers; without the memory for
+// them the context steps with the two sweeps.
+//
+// The rule: FP32 grids of 14 M cells or more whose interior tiles hold 3/8 of
+// the cells (half of them where the H coefficients differ by cell, which costs
+// the fused kernel 16 registers).  The fused pass gains on interior tiles;
+// its general variant, with both half-steps' slab state, does not, and its
+// workgroups are fewer and longer.  Measured, us per step, sweeps / fused:
+// 512x512x256 1086 / 947, 256^3 292 / 281, 320x320x160 292 / 277, magnetic
+// 512x512x128 593 / 574; below the line 224^3 213 / 224, 512x512x64 303 / 314
+// (interior a third), magnetic 256^3 302 / 332, 128x128x64 27 / 36.
+// FDTD_FUSED=0 / 1 overrides it.  Blocks of 16 planes, halved until a launch
+// has 4096 workgroups (256^3: 8 planes 281 us, 16 planes 296).
+void setup_fused(fdtd_ctx *c)
+{
+    const SceneIn &in = c->in;
+    c->fused = false;
+    const char *fv = std::getenv("FDTD_FUSED");
+    const bool force = fv && std::strcmp(fv, "1") == 0;
+    if (in.storage != FDTD_STORE_F32 || (fv && std::strcmp(fv, "0") == 0)) return;
+    const int by = fused_rows(), tx = (in.nx + tile_cols() - 1) / tile_cols(), ty = (in.ny + by - 1) / by;
+    c->kchunk_f = choose_chunks(c, tx * ty, 16, "FDTD_F_PLANES", 4096);
+    sweep_split(c, 2, tile_cols(), by, c->kchunk_f, 1);
+    const int *ib = c->box[2];
+    const double cells = (double)in.nx * in.ny * in.nz;
+    const double inner = (double)(ib[3] - ib[0]) * tile_cols() * (ib[4] - ib[1]) * by * (ib[5] - ib[2]) * c->kchunk_f;
+    if (!force && (cells < 14e6 || inner < (c->h_mode == CLS_UNIFORM ? 0.375 : 0.5) * cells)) return;
+
+    const size_t n_allocs = c->allocs.size();
+    const uint64_t bytes = c->dev_bytes;
+    const std::string err = c->err;
+    int rc = FDTD_OK;
+    for (int f = 0; f < 6 && !rc; ++f) rc = dev_alloc(c, &c->fields2[f], (size_t)c->field_elems * c->esz);
+    for (int p : {0, 1, 4, 5, 8, 9})
+        if (!rc) rc = dev_alloc(c, &c->psi2[p], std::max<size_t>(c->psi_elems[p], 1) * c->esz);
+    if (rc) {
+        while (c->allocs.size() > n_allocs) {
+            (void)hipFree(c->allocs.back());
+            c->allocs.pop_back();
+        }
+        for (auto &f : c->fields2) f = nullptr;
+        for (auto &p : c->psi2) p = nullptr;
+        c->dev_bytes = bytes;
+        c->err = err;
+        return;
+    }
+    c->fused = true;
 }
 
 int do_finalize(fdtd_ctx *c)
@@ -369,8 +433,8 @@ int do_finalize(fdtd_ctx *c)
     // interior / general split of the two sweeps
     {
         const int tcols = c->pair ? pair_tile_cols() : tile_cols();
-        sweep_split(c, 0, tcols, c->pair ? c->pair_kchunk : a.kchunk);
-        sweep_split(c, 1, tcols, c->pair ? c->pair_kchunk : c->kchunk_h);
+        sweep_split(c, 0, tcols, tile_rows(), c->pair ? c->pair_kchunk : a.kchunk);
+        sweep_split(c, 1, tcols, tile_rows(), c->pair ? c->pair_kchunk : c->kchunk_h);
     }
     // psi slabs
     const size_t px_elems = (size_t)in.nz * in.ny * a.Lx;
@@ -405,6 +469,7 @@ int do_finalize(fdtd_ctx *c)
     if ((rc = dev_alloc(c, &tmp, np * nf * sizeof(double2)))) return rc;
     a.dft = (double2 *)tmp;
     if ((rc = upload_tables(c))) return rc;
+    setup_fused(c);
     if ((rc = zero_state(c))) return rc;
     c->finalized = true;
     return FDTD_OK;
@@ -462,6 +527,13 @@ void bind_sets(const fdtd_ctx *c, KArgs &a)
     void **pr[12] = {&a.psi_eyx, &a.psi_ezx, &a.psi_hyx, &a.psi_hzx, &a.psi_exy, &a.psi_ezy,
                      &a.psi_hxy, &a.psi_hzy, &a.psi_exz, &a.psi_eyz, &a.psi_hxz, &a.psi_hyz};
     for (int p = 0; p < 12; ++p) *pr[p] = c->psi[p];
+    if (c->fused) {
+        void **nd[6] = {&a.nex, &a.ney, &a.nez, &a.nhx, &a.nhy, &a.nhz};
+        for (int f = 0; f < 6; ++f) *nd[f] = (char *)c->fields2[f] + g;
+        a.npsi_eyx = c->psi2[0]; a.npsi_ezx = c->psi2[1];
+        a.npsi_exy = c->psi2[4]; a.npsi_ezy = c->psi2[5];
+        a.npsi_exz = c->psi2[8]; a.npsi_eyz = c->psi2[9];
+    }
 }
 
 // One time step m.  base carries the per-call flags (rec, snapshot); the
@@ -475,6 +547,21 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
     a.tiles_y = c->ka.tiles_y;
     a.kchunk = c->pair ? c->pair_kchunk : c->ka.kchunk;
     bind_sets(c, a);
+    if (c->fused && a.lc[3] == 0) {   // (light-cone steps sweep their box in place)
+        a.tiles_x = c->ka.tiles_x;
+        a.tiles_y = (a.ny + fused_rows() - 1) / fused_rows();
+        a.kchunk = c->kchunk_f;
+        for (int q = 0; q < 6; ++q) a.ib[q] = c->box[2][q];
+        a.sub[3] = 0;
+        if (ev0) (void)hipEventRecord(ev0, c->stream);
+        e = launch_step(c->e_mode, c->h_mode, a, m, c->stream);
+        if (ev1) (void)hipEventRecord(ev1, c->stream);
+        if (ev2) (void)hipEventRecord(ev2, c->stream);
+        if (ev3) (void)hipEventRecord(ev3, c->stream);
+        for (int f = 0; f < 6; ++f) std::swap(c->fields[f], c->fields2[f]);
+        for (int p : {0, 1, 4, 5, 8, 9}) std::swap(c->psi[p], c->psi2[p]);
+        return e;
+    }
     auto half = [c](bool efield, int storage, int mode, const KArgs &ka, int mm, hipStream_t st) {
         return c->pair ? launch_pair_half_step(efield, storage, mode, ka, mm, st, c->pair_gen_cells)
                        : launch_half_step(efield, storage, mode, ka, mm, st);

@@ -99,6 +99,11 @@ struct KArgs {
     float *snap;
     int sb[6];
     int snap_base;
+    // where the fused step (fused.hip) writes the fields and the E sweep's
+    // psi: the other buffer of each pair (the host swaps the two after a
+    // step); psi_h is updated in place
+    void *nex, *ney, *nez, *nhx, *nhy, *nhz;
+    void *npsi_eyx, *npsi_ezx, *npsi_exy, *npsi_ezy, *npsi_exz, *npsi_eyz;
 };
 
 // Tile counts of the region variants of a sweep (tile_of_region).

@@ -129,7 +129,8 @@ typedef struct {
     int      storage;            /* FDTD_STORE_*                               */
     double   dt;
     double   last_run_ms;        /* hipEvent time of the last fdtd_run() loop  */
-    double   e_kernel_ms;        /* mean E-kernel launch time (fdtd_profile)   */
+    double   e_kernel_ms;        /* mean E-kernel launch time (fdtd_profile);
+                                    the whole step's where one pass does both */
     double   h_kernel_ms;        /* mean H-kernel launch time (fdtd_profile)   */
     double   step_kernel_ms;     /* mean time of one step's launches            */
     int      interior_split;     /* 1: the sweeps run interior / x-edge /
