@@ -36,6 +36,11 @@ hipError_t launch_pair_half_step(bool efield, int storage, int mode, const KArgs
                                  bool gen_cells);
 hipError_t launch_step(int em, int hm, const KArgs &a, int m, hipStream_t s);
 int fused_rows();
+size_t persist_lds(int units, int sx);
+int persist_max_units();
+bool persist_fits(int storage, int units, int tiles, size_t lds, int device);
+hipError_t launch_persist(int storage, const KArgs &a, const PArgs &p, int tiles, size_t lds, hipStream_t s);
+hipError_t launch_dft(const KArgs &a, int nprobe, int m0, int n, hipStream_t s);
 int tile_rows();
 int tile_cols();
 int pair_tile_cols();
@@ -82,6 +87,12 @@ struct fdtd_ctx {
     int kchunk_f = 0;               // planes per block
     void *fields2[6] = {};
     void *psi2[12] = {};            // (psi_h: null, updated in place)
+    // many steps in one launch (persist.hip): its arguments, tiles, LDS bytes
+    // and the exchange rows' bytes
+    bool persist = false;
+    PArgs pa{};
+    int ptiles = 0;
+    size_t plds = 0, pll = 0;
     double step_ms = 0.0;
     size_t psi_elems[12] = {};
     uint64_t dev_bytes = 0;
@@ -202,6 +213,7 @@ void free_device(fdtd_ctx *c)
     for (auto &q : c->qarr) q = nullptr;
     for (auto &f : c->fields2) f = nullptr;
     for (auto &p : c->psi2) p = nullptr;
+    c->fused = c->persist = false;
 }
 
 // The buffers holding the current state.
@@ -353,6 +365,171 @@ void setup_fused(fdtd_ctx *c)
     c->fused = true;
 }
 
+// Tiles, exchange rows and event lists of the steps in one launch; a context
+// they do not fit, or without the memory, steps with the sweeps.
+//
+// The rule: FP32, FP16 or BF16 storage, one H class, and a tiling of at most
+// 256 tiles of 80 row segments (about 1.3 M cells), each with at most
+// P_MAX_EVENTS source edges and probes.  Every such grid measured is faster in
+// one launch, us per step, sweeps / one launch of 300 steps: 64^3 13.5 / 3.9,
+// 300x60x40 34.7 / 11.3, 110x150x53 27.1 / 15.2, 128x128x64 27.8 / 14.6 (FP16
+// 23.0 / 16.7), 128x128x80 32.8 / 17.1, 12x9x8 10.0 / 3.2; and from few steps:
+// 8 steps of 64^3 13.0 / 7.0, of 128x128x64 28.0 / 19.0 (the launch, loading
+// and storing the tiles take about 25 us).  FDTD_PERSIST=0 turns it off.
+void setup_persist(fdtd_ctx *c)
+{
+    const SceneIn &in = c->in;
+    c->persist = false;
+    const char *ev = std::getenv("FDTD_PERSIST");
+    if (in.storage == FDTD_STORE_BQ16 || c->h_mode != CLS_UNIFORM || c->fused || (ev && std::strcmp(ev, "0") == 0))
+        return;
+    // the tiling: at most one tile per CU and 160 KB of LDS each, the fewest
+    // units (64-cell row segments) per tile, then the fewest rows exchanged
+    const size_t lds_max = 160 * 1024;
+    const int cus = 256, sx = (in.nx + 63) / 64;
+    if ((double)in.ny * in.nz * sx > (double)cus * persist_max_units()) return;
+    int ty = 0, tz = 0;
+    double best = 0.0;
+    for (int z = 1; z <= in.nz && z <= 64; ++z)
+        for (int y = 1; y <= in.ny && y <= 64; ++y) {
+            if (((in.ny + y - 1) / y) * ((in.nz + z - 1) / z) > cus || y * z * sx > persist_max_units() ||
+                persist_lds(y * z * sx, sx) > lds_max)
+                continue;
+            const double cost = y * z * sx + 0.25 * (y + z) * sx;
+            if (ty == 0 || cost < best) {
+                best = cost;
+                ty = y;
+                tz = z;
+            }
+        }
+    if (ty == 0) return;
+    const int gy = (in.ny + ty - 1) / ty, gz = (in.nz + tz - 1) / tz, tiles = gy * gz, U = ty * tz * sx;
+    const size_t lds = persist_lds(U, sx);
+    if (!persist_fits(in.storage, U, tiles, lds, c->device)) return;
+    // events of each tile's units: E events, then (after their terminator) H events
+    const int nx = in.nx, ny = in.ny, nz = in.nz, XS = sx * 64;
+    const int *L = in.cpml.thick;
+    std::vector<std::vector<PEvent>> per((size_t)tiles * 2 * U);
+    int half = 0;
+    for (const Event &e : c->built.events) {
+        if (e.kind < 0) {
+            ++half;
+            continue;
+        }
+        const int i = e.col % nx, j = e.col / nx;
+        const int tile = (e.k / tz) * gy + j / ty, u = ((e.k % tz) * ty + j % ty) * sx + i / 64;
+        PEvent q{i, e.kind, e.id, 0, 0.f, 0.f, 0.f, 0.f};
+        if (e.kind == EV_SOURCE) {
+            const SrcEdge &se = c->built.srcs[e.id];
+            q.wave = se.wave;
+            q.ceze = se.ceze; q.cezhy = se.cezhy; q.cezhx = se.cezhx; q.cezj = se.cezj;
+        }
+        per[((size_t)tile * 2 + half) * U + u].push_back(q);
+    }
+    // exchange rows, [2][XS] words each: H of a tile's last row (hx, hz) and
+    // last plane (hx, hy), E of its first row (ex, ez) and plane (ex, ey)
+    const size_t wj = (size_t)gy * nz * 2 * XS, wk = (size_t)gz * ny * 2 * XS;
+    const size_t o_hj = 0, o_hk = wj, o_ej = wj + wk, o_ek = 2 * wj + wk;
+    std::vector<PTile> pt(tiles);
+    std::vector<PUnit> units[2];
+    std::vector<PEvent> events;
+    for (auto &v : units) v.assign((size_t)tiles * U, PUnit{});
+    for (int t = 0; t < tiles; ++t) {
+        const int tj = t % gy, tk = t / gy, j0 = tj * ty, k0 = tk * tz;
+        const int nyt = std::min(ty, ny - j0), nzt = std::min(tz, nz - k0);
+        pt[t] = PTile{nyt * nzt * sx, (int)events.size(), 0, 0};
+        for (int h = 0; h < 2; ++h) {
+            int n = 0;
+            for (int pass = 0; pass < 2; ++pass)
+                for (int u = 0; u < U; ++u) {
+                    const int jt = (u / sx) % ty, kt = u / sx / ty, j = j0 + jt, k = k0 + kt, i0 = (u % sx) * 64;
+                    if (jt >= nyt || kt >= nzt) continue;
+                    const bool sj = h == 0 ? jt == 0 : jt == nyt - 1, sk = h == 0 ? kt == 0 : kt == nzt - 1;
+                    if ((sj || sk) != (pass == 1)) continue;   // units that wait come last
+                    PUnit q{};
+                    q.lds = u * 6 * 64;
+                    q.i0 = i0;
+                    q.j = j;
+                    q.k = k;
+                    const bool gj = sj && (h == 0 ? j > 0 : j < ny - 1), gk = sk && (h == 0 ? k > 0 : k < nz - 1);
+                    const bool lo = h == 0;   // the E slabs leave out cell 0 (fdtdrav.h:752, 402)
+                    const bool ys = ((!lo || j > 0) && j < L[2]) || (j >= ny - L[3] && j < ny - 1);
+                    const bool zs = ((!lo || k > 0) && k < L[4]) || (k >= nz - L[5] && k < nz - 1);
+                    const bool xs = i0 < L[0] || i0 + 64 > nx - L[1];
+                    const bool xl = h == 0 ? i0 > 0 : i0 + 64 < XS;
+                    q.flags = (j > 0 ? PU_JLO : 0) | (j < ny - 1 ? PU_JHI : 0) | (k > 0 ? PU_KLO : 0) |
+                              (k < nz - 1 ? PU_KHI : 0) | (ys ? PU_YS : 0) | (zs ? PU_ZS : 0) | (xs ? PU_XS : 0) |
+                              (gj ? PU_GJ : 0) | (gk ? PU_GK : 0) | (!sj ? PU_IJ : 0) | (!sk ? PU_IK : 0) |
+                              (xl ? PU_XL : 0);
+                    q.psx = (k * ny + j) * (L[0] + L[1]);
+                    q.psy = (k * (L[2] + L[3]) + (j < L[2] ? j : j - (ny - L[3]) + L[2])) * in.px + i0;
+                    q.psz = ((k < L[4] ? k : k - (nz - L[5]) + L[4]) * ny + j) * in.px + i0;
+                    const int dj = h == 0 ? tj - 1 : tj + 1, dk = h == 0 ? tk - 1 : tk + 1;
+                    auto row = [&](size_t base, int tile_, int len, int at) {
+                        return (int)(base + ((size_t)tile_ * len + at) * 2 * XS + i0);
+                    };
+                    if (gj) {
+                        q.wj = row(h == 0 ? o_hj : o_ej, dj, nz, k);
+                        q.oj = row(h == 0 ? o_ej : o_hj, tj, nz, k);
+                    }
+                    if (gk) {
+                        q.wk = row(h == 0 ? o_hk : o_ek, dk, ny, j);
+                        q.ok = row(h == 0 ? o_ek : o_hk, tk, ny, j);
+                    }
+                    q.ev = (int)events.size() - pt[t].ev;
+                    for (const PEvent &e : per[((size_t)t * 2 + h) * U + u]) events.push_back(e);
+                    q.nev = (int)events.size() - pt[t].ev - q.ev;
+                    units[h][(size_t)t * U + n++] = q;
+                }
+        }
+        pt[t].nev = (int)events.size() - pt[t].ev;
+        if (pt[t].nev > P_MAX_EVENTS) return;
+    }
+
+    const size_t n_allocs = c->allocs.size();
+    const uint64_t bytes = c->dev_bytes;
+    const std::string err = c->err;
+    void *ll = nullptr, *fd = nullptr, *dt = nullptr, *du[2] = {}, *de = nullptr;
+    c->pll = (2 * wj + 2 * wk) * sizeof(std::uint64_t);
+    int rc = c->pll < ((size_t)1 << 31) ? dev_alloc(c, &ll, c->pll) : FDTD_E_UNSUPPORTED;
+    if (!rc) rc = dev_alloc(c, &fd, sizeof(int));
+    if (!rc) rc = upload(c, &dt, pt.data(), pt.size() * sizeof(PTile));
+    for (int h = 0; h < 2 && !rc; ++h) rc = upload(c, &du[h], units[h].data(), units[h].size() * sizeof(PUnit));
+    if (!rc) rc = upload(c, &de, events.data(), events.size() * sizeof(PEvent));
+    if (!rc && (hipMemsetAsync(ll, 0, c->pll, c->stream) != hipSuccess ||
+                hipMemsetAsync(fd, 0, sizeof(int), c->stream) != hipSuccess))
+        rc = FDTD_E_DEVICE;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) rc = FDTD_E_DEVICE;   // (the host vectors go out of scope)
+    if (rc) {
+        (void)hipGetLastError();
+        while (c->allocs.size() > n_allocs) {
+            (void)hipFree(c->allocs.back());
+            c->allocs.pop_back();
+        }
+        c->dev_bytes = bytes;
+        c->err = err;
+        return;
+    }
+    PArgs &p = c->pa;
+    p = PArgs{};
+    p.ty = ty;
+    p.sx = sx;
+    p.units = U;
+    p.cls16 = c->built.mode == CLS_U16 ? 1 : 0;
+    p.epoch = 1;
+    const char *mp = std::getenv("FDTD_PERSIST_POLLS");
+    p.max_polls = mp ? std::atoi(mp) : 1 << 22;   // some seconds
+    p.failed = (int *)fd;
+    p.ll = (std::uint64_t *)ll;
+    p.tiles = (const PTile *)dt;
+    p.units_e = (const PUnit *)du[0];
+    p.units_h = (const PUnit *)du[1];
+    p.events = (const PEvent *)de;
+    c->ptiles = tiles;
+    c->plds = lds;
+    c->persist = true;
+}
+
 int do_finalize(fdtd_ctx *c)
 {
     const SceneIn &in = c->in;
@@ -470,6 +647,7 @@ int do_finalize(fdtd_ctx *c)
     a.dft = (double2 *)tmp;
     if ((rc = upload_tables(c))) return rc;
     setup_fused(c);
+    setup_persist(c);
     if ((rc = zero_state(c))) return rc;
     c->finalized = true;
     return FDTD_OK;
@@ -592,6 +770,44 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
     return e;
 }
 
+// Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
+// and the call enough steps to pay for it.
+constexpr int P_MIN_STEPS = 4;
+hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
+{
+    hipError_t e = hipSuccess;
+    if (!c->persist || base.lc[3] > 0 || n < P_MIN_STEPS) {
+        for (int m = m0; m < m0 + n && e == hipSuccess; ++m) e = do_step(c, base, m);
+        return e;
+    }
+    PArgs &p = c->pa;
+    if (p.epoch > 0xFFFFFFFFu - (std::uint32_t)n - 2u) {   // the step numbers run out: start over
+        if ((e = hipMemsetAsync(p.ll, 0, c->pll, c->stream)) != hipSuccess) return e;
+        p.epoch = 1;
+    }
+    KArgs a = base;
+    bind_sets(c, a);
+    p.m0 = m0;
+    p.n = n;
+    if ((e = launch_persist(c->in.storage, a, p, c->ptiles, c->plds, c->stream)) != hipSuccess) return e;
+    p.epoch += (std::uint32_t)n + 1u;
+    return a.rec ? launch_dft(a, (int)c->in.probes.size(), m0, n, c->stream) : hipSuccess;
+}
+
+// After a synchronisation: whether a launch of advance gave up a wait.
+int check_advance(fdtd_ctx *c)
+{
+    if (!c->persist) return FDTD_OK;
+    int failed = 0;
+    HIPCHK(c, hipMemcpy(&failed, c->pa.failed, sizeof failed, hipMemcpyDeviceToHost));
+    if (!failed) return FDTD_OK;
+    HIPCHK(c, hipMemset(c->pa.failed, 0, sizeof failed));
+    HIPCHK(c, hipMemset(c->pa.ll, 0, c->pll));
+    c->pa.epoch = 1;
+    return fail(c, FDTD_E_DEVICE, "a workgroup waited too long for a neighbour's rows; the state is not valid "
+                "(fdtd_reset starts over)");
+}
+
 // A stream of one call, drained and destroyed on every return path.
 struct StreamGuard {
     hipStream_t s = nullptr;
@@ -628,18 +844,15 @@ int run_steps(fdtd_ctx *c, int nsteps, bool profile)
     hipEvent_t *evs = all.v.data() + 2;
     const int m0 = c->steps_done;
     HIPCHK(c, hipEventRecord(t0, c->stream));
-    for (int s = 0; s < nsteps; ++s) {
-        const int m = m0 + s;
-        if (profile)
-            HIPCHK(c, do_step(c, c->ka, m, evs[4 * s + 0], evs[4 * s + 1], evs[4 * s + 2], evs[4 * s + 3]));
-        else
-            HIPCHK(c, do_step(c, c->ka, m));
-    }
+    if (!profile) HIPCHK(c, advance(c, c->ka, m0, nsteps));
+    for (int s = 0; profile && s < nsteps; ++s)
+        HIPCHK(c, do_step(c, c->ka, m0 + s, evs[4 * s + 0], evs[4 * s + 1], evs[4 * s + 2], evs[4 * s + 3]));
     HIPCHK(c, hipEventRecord(t1, c->stream));
     HIPCHK(c, hipEventSynchronize(t1));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, t0, t1));
     c->last_run_ms = ms;
+    if (int rc = check_advance(c)) return rc;
     if (profile && nsteps > 0) {
         double se = 0, sh = 0;
         for (int s = 0; s < nsteps; ++s) {
@@ -962,8 +1175,13 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     EventSet sync;
     hipStream_t rs = c->stream;
     if (nseg > 1) {
-        HIPCHK(c, hipStreamCreateWithFlags(&rsg.s, hipStreamNonBlocking));
-        rs = rsg.s;
+        // (a recompute in one launch holds every CU's LDS: beside it the
+        // reverse sweeps slow down by more than it hides, so it runs before
+        // them on the one stream)
+        if (!c->persist) {
+            HIPCHK(c, hipStreamCreateWithFlags(&rsg.s, hipStreamNonBlocking));
+            rs = rsg.s;
+        }
         sync.v.assign(4, nullptr);
         for (auto &e : sync.v) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
@@ -986,13 +1204,14 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     fa.rec = 1;
     fa.snap = nseg == 1 ? hist : nullptr;
     fa.snap_base = 0;
-    for (int m = 0; m < n; ++m) {
-        if (nseg > 1 && m % Kseg == 0 && m > 0)
+    for (int m = 0; m < n; m += Kseg) {
+        if (nseg > 1 && m > 0)
             if ((rc = copy_state(c, pool + (size_t)(m / Kseg - 1) * ck_bytes, true))) return rc;
-        HIPCHK(c, do_step(c, fa, m));
+        HIPCHK(c, advance(c, fa, m, std::min(Kseg, n - m)));
     }
     HIPCHK(c, hipEventRecord(t1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    if ((rc = check_advance(c))) return rc;
     c->steps_done = n;
     // ---- objective J = sum w |X|^2 and dJ/ds[m] = sum w 2 Re(conj(X) phasor[m])
     std::vector<double> X((size_t)np * nf * 2);
@@ -1026,7 +1245,8 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     // first box for every step.  Cells outside it keep stale values, and every
     // segment restarts from a full checkpoint.
     const char *lce = std::getenv("FDTD_LIGHTCONE");
-    const bool lc_on = nseg > 1 && !(lce && std::strcmp(lce, "0") == 0);
+    // (a grid that steps in one launch recomputes whole: cheaper than the box's sweeps)
+    const bool lc_on = nseg > 1 && !c->persist && !(lce && std::strcmp(lce, "0") == 0);
     const bool lc_fixed = lce && std::strcmp(lce, "fixed") == 0;
     // the box dilated by R, or all zero (the whole grid)
     auto cone = [&](int R, int lc[6]) {
@@ -1058,12 +1278,14 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
         cone(Kseg + 2, ra.lc);
         bind_sets(c, ra);
         HIPCHK(c, launch_snap(in.storage, ra, hbuf[q], 0, c->stream));
-        for (int m = s0; m < s1; ++m) {
+        for (int m = s0, runs = 0; m < s1; m += runs) {
+            runs = 1;
             // the cone narrows a cell per step: step m feeds only the
             // snapshots of steps m .. s1-1, so the design box dilated by
             // s1 - m + 2 (Kseg + 2 at most) suffices
             if (!lc_fixed) cone(s1 - m + 2, ra.lc);
-            HIPCHK(c, do_step(c, ra, m));
+            if (c->persist && ra.lc[3] == 0) runs = s1 - m;   // whole-grid steps, one launch
+            HIPCHK(c, advance(c, ra, m, runs));
         }
         HIPCHK(c, hipEventRecord(sync.v[q], c->stream));   // buffer q ready
         return FDTD_OK;
@@ -1107,6 +1329,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     }
     HIPCHK(c, hipEventRecord(t2, c->stream));
     HIPCHK(c, hipEventSynchronize(t2));
+    if ((rc = check_advance(c))) return rc;
     float ms1 = 0.f, ms2 = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms1, t0, t1));
     HIPCHK(c, hipEventElapsedTime(&ms2, t0, t2));

@@ -106,6 +106,45 @@ struct KArgs {
     void *npsi_eyx, *npsi_ezx, *npsi_exy, *npsi_ezy, *npsi_exz, *npsi_eyz;
 };
 
+// Steps of a small grid in one launch (persist.hip).  An event of a unit:
+// its cell i, kind and id as Event, and its source edge's record.
+struct PEvent {
+    int lane, kind, id, wave;
+    float ceze, cezhy, cezhx, cezj;
+};
+constexpr int P_MAX_EVENTS = 96;   // of one tile
+// Flags of a unit: j > 0, j < ny-1, k > 0, k < nz-1; in a y / z slab of the
+// half-step, with lanes in an x slab; the y / z neighbour row belongs to
+// another tile (G: waited for, and an own row posted) or to this one (I);
+// the x-neighbour of lane 0 (E) or 63 (H) lies in the segment beside it.
+enum {
+    PU_JLO = 1, PU_JHI = 2, PU_KLO = 4, PU_KHI = 8, PU_YS = 16, PU_ZS = 32, PU_XS = 64, PU_GJ = 128, PU_GK = 256,
+    PU_IJ = 512, PU_IK = 1024, PU_XL = 2048
+};
+struct PUnit {
+    int lds, flags;         // float offset of the unit in LDS
+    int i0, j, k;
+    int psx, psy, psz;      // psi elements: of the row's cell 0 (x), of cell i0 (y, z)
+    int wj, wk, oj, ok;     // exchange words of cell i0: of the rows waited for, of the rows posted
+    int ev, nev;            // events among the tile's
+    int pad[2];
+};
+struct PTile {
+    int nu, ev, nev, pad;   // units; events
+};
+struct PArgs {
+    int ty, sx, units;         // rows of a tile along y, segments of a row, units of a full tile
+    int cls16;                 // 16-bit class map
+    int m0, n;                 // first step, steps
+    std::uint32_t epoch;       // step number that the rows exchanged before the first step carry
+    int max_polls;             // reads of a row before a wait is given up
+    int *failed;               // raised by a wait that was
+    std::uint64_t *ll;         // words of value and step number of the rows exchanged
+    const PTile *tiles;
+    const PUnit *units_e, *units_h;   // [tile][units], in the half-step's order
+    const PEvent *events;
+};
+
 // Tile counts of the region variants of a sweep (tile_of_region).
 inline void region_tiles(const KArgs &a, int &n_in, int &n_x, int &n_z, int &n_gen)
 {
