@@ -250,6 +250,7 @@ int zero_state(fdtd_ctx *c)
 }
 
 // Upload the material-dependent tables (class map, E/H tables, sources).
+void bind_sets(const fdtd_ctx *c, KArgs &a);
 int upload_tables(fdtd_ctx *c);
 
 // Planes per z-march block.  Many short marches keep every CU's wave slots
@@ -500,7 +501,7 @@ void setup_persist(fdtd_ctx *c)
                 hipMemsetAsync(fd, 0, sizeof(int), c->stream) != hipSuccess))
         rc = FDTD_E_DEVICE;
     if (hipStreamSynchronize(c->stream) != hipSuccess) rc = FDTD_E_DEVICE;   // (the host vectors go out of scope)
-    if (rc) {
+    auto drop = [&]() {
         (void)hipGetLastError();
         while (c->allocs.size() > n_allocs) {
             (void)hipFree(c->allocs.back());
@@ -508,8 +509,8 @@ void setup_persist(fdtd_ctx *c)
         }
         c->dev_bytes = bytes;
         c->err = err;
-        return;
-    }
+    };
+    if (rc) return drop();
     PArgs &p = c->pa;
     p = PArgs{};
     p.ty = ty;
@@ -527,6 +528,16 @@ void setup_persist(fdtd_ctx *c)
     p.events = (const PEvent *)de;
     c->ptiles = tiles;
     c->plds = lds;
+    // A launch of no steps (it stores the state that it read): cooperative
+    // launches are refused while another process on the card has made some,
+    // and the sweeps are used then.
+    KArgs ka = c->ka;
+    bind_sets(c, ka);
+    ka.snap = nullptr;
+    if (launch_persist(in.storage, ka, p, tiles, lds, c->stream) != hipSuccess ||
+        hipStreamSynchronize(c->stream) != hipSuccess)
+        return drop();
+    p.epoch += 1;
     c->persist = true;
 }
 
