@@ -40,6 +40,10 @@ size_t persist_lds(int units, int sx);
 int persist_max_units();
 bool persist_fits(int storage, int units, int tiles, size_t lds, int device);
 hipError_t launch_persist(int storage, const KArgs &a, const PArgs &p, int tiles, size_t lds, hipStream_t s);
+size_t adj_persist_lds(int units, int sx, int events);
+int adj_persist_max_units();
+bool adj_persist_fits(int units, int tiles, size_t lds, int device);
+hipError_t launch_adj_persist(const KArgs &a, const AArgs &b, const RArgs &p, int tiles, size_t lds, hipStream_t s);
 hipError_t launch_dft(const KArgs &a, int nprobe, int m0, int n, hipStream_t s);
 int tile_rows();
 int tile_cols();
@@ -93,6 +97,10 @@ struct fdtd_ctx {
     PArgs pa{};
     int ptiles = 0;
     size_t plds = 0, pll = 0;
+    // reverse steps likewise (adj_persist.hip; on persist's tiles and rows)
+    bool radj = false;
+    RArgs ra{};
+    size_t rlds = 0;
     double step_ms = 0.0;
     size_t psi_elems[12] = {};
     uint64_t dev_bytes = 0;
@@ -213,7 +221,7 @@ void free_device(fdtd_ctx *c)
     for (auto &q : c->qarr) q = nullptr;
     for (auto &f : c->fields2) f = nullptr;
     for (auto &p : c->psi2) p = nullptr;
-    c->fused = c->persist = false;
+    c->fused = c->persist = c->radj = false;
 }
 
 // The buffers holding the current state.
@@ -366,6 +374,169 @@ void setup_fused(fdtd_ctx *c)
     c->fused = true;
 }
 
+// Reverse steps in one launch: on the tiles of the forward ones (ty x tz rows
+// of sx segments, gy of them along y), whose exchange rows are taken from the
+// forward units.  Rule: wherever the forward steps run in one launch and a
+// tile's units and events fit 160 KB of LDS (76 units; any storage form: the
+// reverse state is FP32).  All of it is faster that way; a reverse step, us,
+// launched / in one launch: 28x24x22 14.3 / 5.3, 64^3 18.4 / 5.9, 127x100x50
+// 32.6 / 14.0, 300x60x40 54.0 / 17.1, 128x128x64 47.0 / 21.1, 112x96x90 46.1 /
+// 28.0, 96^3 43.6 / 26.8.  FDTD_ADJ_PERSIST=0 turns it off.
+void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector<PUnit> (&units)[2], int gy, int tz)
+{
+    const SceneIn &in = c->in;
+    const Built &bt = c->built;
+    const int nx = in.nx, ny = in.ny, nz = in.nz, ty = c->pa.ty, sx = c->pa.sx, U = c->pa.units;
+    const char *ev = std::getenv("FDTD_ADJ_PERSIST");
+    if ((ev && std::strcmp(ev, "0") == 0) || U > adj_persist_max_units() || sx >= 1 << (31 - RU_SEG) || ny > 0xFFFF ||
+        nz > 0xFFFF)
+        return;
+    // a tile's units: those on its high sides first, on its low sides last
+    // (high and low: last); at[u]: where unit u comes
+    const int tiles = c->ptiles;
+    std::vector<RUnit> ru((size_t)tiles * U, RUnit{});
+    std::vector<PTile> pt(ptiles);
+    std::vector<const PUnit *> pe(U), ph(U);
+    std::vector<std::vector<REvent>> le(U), lh(U);   // a tile's events, by unit
+    std::vector<REvent> events;
+    int max_ev = 0;
+    // E events and source edges by tile
+    struct At { int i, j, k, u; Event e; };
+    std::vector<std::vector<At>> per(tiles);
+    auto tile_of = [&](int j, int k) { return (k / tz) * gy + j / ty; };
+    auto unit_of = [&](int i, int j, int k) { return ((k % tz) * ty + j % ty) * sx + i / 64; };
+    for (const Event &e : bt.events) {
+        if (e.kind < 0) break;   // (the H events follow)
+        if (e.kind != EV_SOURCE && e.kind > EV_PROBE + 2) continue;
+        const int i = e.col % nx, j = e.col / nx;
+        per[tile_of(j, e.k)].push_back(At{i, j, e.k, unit_of(i, j, e.k), e});
+    }
+    // source gathers: of the cell itself, of (i-1, j) and of (i, j-1), the
+    // latter in the tile below when j is its first row
+    std::vector<std::vector<std::pair<int, REvent>>> gather(tiles);
+    std::vector<char> third((size_t)ny * nz * sx, 0);   // rows (by segment) posted with dJ/dEz
+    for (int q = 0; q < 3; ++q)
+        for (int t = 0; t < tiles; ++t)
+            for (const At &s : per[t]) {
+                if (s.e.kind != EV_SOURCE) continue;
+                const int i = q == 1 ? s.i - 1 : s.i, j = q == 2 ? s.j - 1 : s.j;
+                if (i < 0 || j < 0) continue;
+                const SrcEdge &se = bt.srcs_si[s.e.id];
+                size_t cl = 0;
+                if (!bt.e_uniform && !bt.cls.empty()) cl = bt.cls[((size_t)s.k * ny + s.j) * in.px + s.i];
+                const float *ez = bt.etab_si.data() + (cl * 3 + 2) * 4;
+                const int *L = in.cpml.thick;
+                auto slab = [](int v, int n, int lo, int hi) { return (v > 0 && v < lo) || (v >= n - hi && v < n - 1); };
+                const float kx = slab(s.i, nx, L[0], L[1]) ? bt.prof[0][4 * (size_t)s.i + 2] : 1.0f;
+                const float ky = slab(s.j, ny, L[2], L[3]) ? bt.prof[1][4 * (size_t)s.j + 2] : 1.0f;
+                const int to = tile_of(j, s.k);
+                REvent r{i, q, to == t ? (int)(&s - per[t].data()) : -1, 0, se.cezhy, se.cezhx, ez[1] / kx, ez[2] / ky};
+                if (to != t) third[((size_t)s.k * ny + s.j) * sx + s.i / 64] = 1;
+                gather[to].push_back({unit_of(i, j, s.k), r});
+            }
+    for (int t = 0; t < tiles; ++t) {
+        std::fill(pe.begin(), pe.end(), nullptr);
+        std::fill(ph.begin(), ph.end(), nullptr);
+        const int nu = ptiles[t].nu;
+        for (int n = 0; n < nu; ++n) {
+            const PUnit &e = units[0][(size_t)t * U + n], &h = units[1][(size_t)t * U + n];
+            pe[e.lds / (6 * 64)] = &e;
+            ph[h.lds / (6 * 64)] = &h;
+        }
+        pt[t].ev = (int)events.size();
+        std::vector<int> where(per[t].size());   // of each E event
+        std::vector<int> evw(U, 0), hvw(U, 0);
+        for (int u = 0; u < U; ++u) {
+            const int first = (int)events.size() - pt[t].ev;
+            for (size_t x = 0; x < per[t].size(); ++x) {
+                const At &s = per[t][x];
+                if (s.u != u) continue;
+                where[x] = (int)events.size() - pt[t].ev;
+                const float c0 = s.e.kind == EV_SOURCE ? bt.srcs_si[s.e.id].ceze : 0.f;
+                events.push_back(REvent{s.i, s.e.kind, s.e.id, 0, c0, 0.f, 0.f, 0.f});
+            }
+            evw[u] = first | ((int)events.size() - pt[t].ev - first) << 16;
+        }
+        for (int u = 0; u < U; ++u) {
+            const int first = (int)events.size() - pt[t].ev;
+            for (const auto &g : gather[t]) {
+                if (g.first != u) continue;
+                events.push_back(g.second);
+                if (g.second.id >= 0) events.back().id = where[g.second.id];
+            }
+            hvw[u] = first | ((int)events.size() - pt[t].ev - first) << 16;
+        }
+        pt[t].nev = (int)events.size() - pt[t].ev;
+        if (pt[t].nev > 0x7FFF) return;   // (16-bit fields of RUnit)
+        max_ev = std::max(max_ev, pt[t].nev);
+        int n = 0;
+        for (int pass = 0; pass < 3; ++pass)
+            for (int u = 0; u < U; ++u) {
+                if (!pe[u]) continue;
+                const PUnit &e = *pe[u], &h = *ph[u];
+                const bool lo = !(e.flags & PU_IJ) || !(e.flags & PU_IK), hi = !(h.flags & PU_IJ) || !(h.flags & PU_IK);
+                if ((lo ? 2 : hi ? 0 : 1) != pass) continue;
+                auto f = [](int from, int bit, int to) { return from & bit ? to : 0; };
+                // (third words: of rows that another tile waits for)
+                const bool se = (e.flags & PU_GJ) && third[((size_t)e.k * ny + e.j) * sx + e.i0 / 64];
+                const bool sh = (h.flags & PU_GJ) && third[((size_t)h.k * ny + h.j + 1) * sx + h.i0 / 64];
+                RUnit &r = ru[(size_t)t * U + n++];
+                r.w[RW_UNIT] = u;
+                r.w[RW_FLAGS] = f(e.flags, PU_JLO, RU_JLO) | f(e.flags, PU_JHI, RU_JHI) | f(e.flags, PU_KLO, RU_KLO) |
+                                f(e.flags, PU_KHI, RU_KHI) | f(e.flags, PU_XS, RU_XS) | f(e.flags, PU_YS, RU_YSE) |
+                                f(h.flags, PU_YS, RU_YSH) | f(e.flags, PU_ZS, RU_ZSE) | f(h.flags, PU_ZS, RU_ZSH) |
+                                f(e.flags, PU_GJ, RU_GJE) | f(e.flags, PU_GK, RU_GKE) | f(h.flags, PU_GJ, RU_GJH) |
+                                f(h.flags, PU_GK, RU_GKH) | f(e.flags, PU_IJ, RU_IJE) | f(e.flags, PU_IK, RU_IKE) |
+                                f(h.flags, PU_IJ, RU_IJH) | f(h.flags, PU_IK, RU_IKH) | f(e.flags, PU_XL, RU_XLE) |
+                                f(h.flags, PU_XL, RU_XLH) | (se ? RU_SRE : 0) | (sh ? RU_SRH : 0) |
+                                (int)((unsigned)(e.i0 / 64) << RU_SEG);
+                r.w[RW_JK] = (int)((unsigned)e.j | (unsigned)e.k << 16);
+                r.w[RW_PSX] = e.psx;
+                r.w[RW_PSY] = e.psy;
+                r.w[RW_PSZ] = e.psz;
+                r.w[RW_WJE] = e.wj; r.w[RW_WKE] = e.wk; r.w[RW_OJE] = e.oj; r.w[RW_OKE] = e.ok;
+                r.w[RW_WJH] = h.wj; r.w[RW_WKH] = h.wk; r.w[RW_OJH] = h.oj; r.w[RW_OKH] = h.ok;
+                r.w[RW_EVE] = evw[u];
+                r.w[RW_EVH] = hvw[u];
+            }
+    }
+    const size_t lds = adj_persist_lds(U, sx, max_ev);
+    if (lds > 160 * 1024 || !adj_persist_fits(U, c->ptiles, lds, c->device)) return;
+    const size_t n_allocs = c->allocs.size();
+    const uint64_t bytes = c->dev_bytes;
+    const std::string err = c->err;
+    void *dt = nullptr, *du = nullptr, *de = nullptr;
+    int rc = upload(c, &dt, pt.data(), pt.size() * sizeof(PTile));
+    if (!rc) rc = upload(c, &du, ru.data(), ru.size() * sizeof(RUnit));
+    if (!rc) rc = upload(c, &de, events.data(), events.size() * sizeof(REvent));
+    if (hipStreamSynchronize(c->stream) != hipSuccess) rc = FDTD_E_DEVICE;   // (the host vectors go out of scope)
+    if (rc) {
+        (void)hipGetLastError();
+        while (c->allocs.size() > n_allocs) {
+            (void)hipFree(c->allocs.back());
+            c->allocs.pop_back();
+        }
+        c->dev_bytes = bytes;
+        c->err = err;
+        return;
+    }
+    RArgs &r = c->ra;
+    r = RArgs{};
+    r.ty = ty;
+    r.sx = sx;
+    r.units = U;
+    r.cls16 = c->pa.cls16;
+    r.euni = bt.e_uniform ? 1 : 0;
+    r.max_polls = c->pa.max_polls;
+    r.failed = c->pa.failed;
+    r.ll = c->pa.ll;
+    r.tiles = (const PTile *)dt;
+    r.u = (const RUnit *)du;
+    r.events = (const REvent *)de;
+    c->rlds = lds;
+    c->radj = true;
+}
+
 // Tiles, exchange rows and event lists of the steps in one launch; a context
 // they do not fit, or without the memory, steps with the sweeps.
 //
@@ -380,7 +551,7 @@ void setup_fused(fdtd_ctx *c)
 void setup_persist(fdtd_ctx *c)
 {
     const SceneIn &in = c->in;
-    c->persist = false;
+    c->persist = c->radj = false;
     const char *ev = std::getenv("FDTD_PERSIST");
     if (in.storage == FDTD_STORE_BQ16 || c->h_mode != CLS_UNIFORM || c->fused || (ev && std::strcmp(ev, "0") == 0))
         return;
@@ -428,9 +599,10 @@ void setup_persist(fdtd_ctx *c)
         per[((size_t)tile * 2 + half) * U + u].push_back(q);
     }
     // exchange rows, [2][XS] words each: H of a tile's last row (hx, hz) and
-    // last plane (hx, hy), E of its first row (ex, ez) and plane (ex, ey)
-    const size_t wj = (size_t)gy * nz * 2 * XS, wk = (size_t)gz * ny * 2 * XS;
-    const size_t o_hj = 0, o_hk = wj, o_ej = wj + wk, o_ek = 2 * wj + wk;
+    // last plane (hx, hy), E of its first row (ex, ez; [3][XS], the third for
+    // the reverse steps) and plane (ex, ey)
+    const size_t wj = (size_t)gy * nz * XS, wk = (size_t)gz * ny * XS;
+    const size_t o_hj = 0, o_hk = 2 * wj, o_ej = o_hk + 2 * wk, o_ek = o_ej + 3 * wj, words = o_ek + 2 * wk;
     std::vector<PTile> pt(tiles);
     std::vector<PUnit> units[2];
     std::vector<PEvent> events;
@@ -466,16 +638,18 @@ void setup_persist(fdtd_ctx *c)
                     q.psy = (k * (L[2] + L[3]) + (j < L[2] ? j : j - (ny - L[3]) + L[2])) * in.px + i0;
                     q.psz = ((k < L[4] ? k : k - (nz - L[5]) + L[4]) * ny + j) * in.px + i0;
                     const int dj = h == 0 ? tj - 1 : tj + 1, dk = h == 0 ? tk - 1 : tk + 1;
-                    auto row = [&](size_t base, int tile_, int len, int at) {
-                        return (int)(base + ((size_t)tile_ * len + at) * 2 * XS + i0);
-                    };
+                    // of a tile in y (in z), the row in plane k (the row j) from cell i0
+                    auto hj = [&](int tile_) { return (int)(o_hj + ((size_t)tile_ * nz + k) * 2 * XS + i0); };
+                    auto ej = [&](int tile_) { return (int)(o_ej + ((size_t)tile_ * nz + k) * 3 * XS + i0); };
+                    auto hk = [&](int tile_) { return (int)(o_hk + ((size_t)tile_ * ny + j) * 2 * XS + i0); };
+                    auto ek = [&](int tile_) { return (int)(o_ek + ((size_t)tile_ * ny + j) * 2 * XS + i0); };
                     if (gj) {
-                        q.wj = row(h == 0 ? o_hj : o_ej, dj, nz, k);
-                        q.oj = row(h == 0 ? o_ej : o_hj, tj, nz, k);
+                        q.wj = h == 0 ? hj(dj) : ej(dj);
+                        q.oj = h == 0 ? ej(tj) : hj(tj);
                     }
                     if (gk) {
-                        q.wk = row(h == 0 ? o_hk : o_ek, dk, ny, j);
-                        q.ok = row(h == 0 ? o_ek : o_hk, tk, ny, j);
+                        q.wk = h == 0 ? hk(dk) : ek(dk);
+                        q.ok = h == 0 ? ek(tk) : hk(tk);
                     }
                     q.ev = (int)events.size() - pt[t].ev;
                     for (const PEvent &e : per[((size_t)t * 2 + h) * U + u]) events.push_back(e);
@@ -491,7 +665,7 @@ void setup_persist(fdtd_ctx *c)
     const uint64_t bytes = c->dev_bytes;
     const std::string err = c->err;
     void *ll = nullptr, *fd = nullptr, *dt = nullptr, *du[2] = {}, *de = nullptr;
-    c->pll = (2 * wj + 2 * wk) * sizeof(std::uint64_t);
+    c->pll = words * sizeof(std::uint64_t);
     int rc = c->pll < ((size_t)1 << 31) ? dev_alloc(c, &ll, c->pll) : FDTD_E_UNSUPPORTED;
     if (!rc) rc = dev_alloc(c, &fd, sizeof(int));
     if (!rc) rc = upload(c, &dt, pt.data(), pt.size() * sizeof(PTile));
@@ -539,6 +713,7 @@ void setup_persist(fdtd_ctx *c)
         return drop();
     p.epoch += 1;
     c->persist = true;
+    if (!in.design_eps.empty()) setup_radj(c, pt, units, gy, tz);
 }
 
 int do_finalize(fdtd_ctx *c)
@@ -784,6 +959,15 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
 // Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
 // and the call enough steps to pay for it.
 constexpr int P_MIN_STEPS = 4;
+
+// Before a launch of n steps: start over when the step numbers run out.
+hipError_t new_epochs(fdtd_ctx *c, int n)
+{
+    if (c->pa.epoch <= 0xFFFFFFFFu - (std::uint32_t)n - 2u) return hipSuccess;
+    c->pa.epoch = 1;
+    return hipMemsetAsync(c->pa.ll, 0, c->pll, c->stream);
+}
+
 hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
 {
     hipError_t e = hipSuccess;
@@ -792,10 +976,7 @@ hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
         return e;
     }
     PArgs &p = c->pa;
-    if (p.epoch > 0xFFFFFFFFu - (std::uint32_t)n - 2u) {   // the step numbers run out: start over
-        if ((e = hipMemsetAsync(p.ll, 0, c->pll, c->stream)) != hipSuccess) return e;
-        p.epoch = 1;
-    }
+    if ((e = new_epochs(c, n)) != hipSuccess) return e;
     KArgs a = base;
     bind_sets(c, a);
     p.m0 = m0;
@@ -1023,6 +1204,10 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     const int n = n_steps;
     const int bx = dnx + 1, by = dny + 1, bz = dnz + 1;
     const i64 nb = (i64)bx * by * bz;
+    // all reverse steps of a segment in one launch (a switch of the launched
+    // sweeps asks for those)
+    const bool radj = c->radj && !std::getenv("FDTD_ADJ_GATHER") && !std::getenv("FDTD_ADJ_CHUNKS") &&
+                      !std::getenv("FDTD_INTERIOR");
     // adjoint fields (6) and, on narrow grids, every cell's transposed
     // quantities (12 arrays), guard planes included
     const int nq = adj_stores_quantities(nx) ? 12 : 0;
@@ -1084,7 +1269,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
         b.ebn[q] = b.eb[q];   // in place unless the fused interior sweep is set up below
         b.hbn[q] = b.hb[q];
     }
-    for (int q = 0; q < nq; ++q) {
+    for (int q = 0; q < (radj ? 0 : nq); ++q) {   // (one launch keeps them in LDS)
         char *t = (char *)mem.get((size_t)c->field_elems * 4);
         if (!t) return fail(c, FDTD_E_NOMEM, "adjoint transposed-quantity allocation failed");
         HIPCHK(c, hipMemsetAsync(t, 0, (size_t)c->field_elems * 4, c->stream));
@@ -1307,7 +1492,16 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
         if (nseg > 1) HIPCHK(c, hipStreamWaitEvent(rs, sync.v[q], 0));
         b.hist = hbuf[q];
         b.hist_base = s0;
-        for (int m = s1 - 1; m >= s0; --m) {
+        if (radj) {
+            RArgs &r = c->ra;
+            HIPCHK(c, new_epochs(c, s1 - s0));
+            r.m1 = s1 - 1;
+            r.n = s1 - s0;
+            r.epoch = c->pa.epoch;
+            HIPCHK(c, launch_adj_persist(aa, b, r, c->ptiles, c->rlds, rs));
+            c->pa.epoch += (std::uint32_t)r.n + 1u;
+        }
+        for (int m = s1 - 1; !radj && m >= s0; --m) {
             const int fst = m < s1 - 1 ? m + 1 : -1;
             if (pp) {
                 const hipStream_t fs = fz_async ? fsg.s : rs;
@@ -1327,7 +1521,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
                 HIPCHK(c, launch_adj(1, mode, euni, huni, aa, b, m, -1, 1, rs));
             }
         }
-        HIPCHK(c, launch_adj(0, mode, euni, huni, aa, b, s0, s0, 0, rs));
+        if (!radj) HIPCHK(c, launch_adj(0, mode, euni, huni, aa, b, s0, s0, 0, rs));
         if (pp) swap_e();
         if (nseg > 1) {
             HIPCHK(c, hipEventRecord(sync.v[2 + q], rs));   // buffer q free

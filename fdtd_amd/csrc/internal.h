@@ -145,6 +145,46 @@ struct PArgs {
     const PEvent *events;
 };
 
+// Reverse steps of a small grid in one launch (adj_persist.hip), on the same
+// tiles and exchange rows.  A unit is 16 words: its place in LDS, flags, j and
+// k << 16, psi elements as PUnit, exchange words of the E and the H half-step
+// (rows waited for, rows posted), and its events (first, number << 16).
+enum {
+    RW_UNIT, RW_FLAGS, RW_JK, RW_PSX, RW_PSY, RW_PSZ, RW_WJE, RW_WKE, RW_OJE, RW_OKE, RW_WJH, RW_WKH, RW_OJH, RW_OKH,
+    RW_EVE, RW_EVH
+};
+struct RUnit {
+    int w[16];
+};
+// Flags as PU_*, those that differ for the E and the H half-step twice; RU_SR:
+// the row posted (E) or waited for (H) holds source edges, and a third value.
+// The bits from RU_SEG: the segment of the row.
+enum {
+    RU_JLO = 1, RU_JHI = 2, RU_KLO = 4, RU_KHI = 8, RU_XS = 16, RU_YSE = 32, RU_YSH = 64, RU_ZSE = 128, RU_ZSH = 256,
+    RU_GJE = 512, RU_GKE = 1 << 10, RU_GJH = 1 << 11, RU_GKH = 1 << 12, RU_IJE = 1 << 13, RU_IKE = 1 << 14,
+    RU_IJH = 1 << 15, RU_IKH = 1 << 16, RU_XLE = 1 << 17, RU_XLH = 1 << 18, RU_SRE = 1 << 19, RU_SRH = 1 << 20,
+    RU_SEG = 21
+};
+// E half-step: a source edge (c0: its own Ez coefficient; c1 receives its
+// dJ/dEz) or an E probe (id).  H half-step: a source edge gathered by the cell,
+// kind 0 on it, 1 at (i+1, j), 2 at (i, j+1); id: its E event in this tile or
+// -1; c0, c1: its curl coefficients, c2, c3: the material's it replaces.
+struct REvent {
+    int lane, kind, id, pad;
+    float c0, c1, c2, c3;
+};
+struct RArgs {
+    int ty, sx, units, cls16, euni;
+    int m1, n;                 // last step, steps
+    std::uint32_t epoch;
+    int max_polls;
+    int *failed;
+    std::uint64_t *ll;
+    const PTile *tiles;
+    const RUnit *u;            // [tile][units]
+    const REvent *events;
+};
+
 // Tile counts of the region variants of a sweep (tile_of_region).
 inline void region_tiles(const KArgs &a, int &n_in, int &n_x, int &n_z, int &n_gen)
 {

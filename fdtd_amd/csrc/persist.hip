@@ -37,55 +37,10 @@
 
 #include "device_common.h"
 #include "internal.h"
+#include "persist_common.h"
 #include "sweep_common.h"
 
 namespace fdtd {
-
-typedef std::uint32_t u32;
-typedef std::uint64_t u64;
-
-constexpr int PW = 16;   // waves per workgroup
-
-__device__ __forceinline__ void ll_put(u64 *p, float v, u32 tag)
-{
-    __hip_atomic_store(p, (u64)__float_as_uint(v) | ((u64)tag << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ u64 ll_get(const u64 *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float ll_val(u64 w) { return __uint_as_float((u32)w); }
-__device__ __forceinline__ bool ll_is(u64 w, u32 tag) { return (u32)(w >> 32) == tag; }
-
-// The words at pa, pa + n (when ga) and pb, pb + n (when gb), once all of
-// them carry `tag` on every lane of the wave (ga and gb are wave-uniform).
-__device__ __forceinline__ void ll_wait(const PArgs &p, bool ga, const u64 *pa, bool gb, const u64 *pb, int n, u32 tag,
-                                        bool &dead, float &a0, float &a1, float &b0, float &b1)
-{
-    u64 w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-    for (int t = 0;; ++t) {
-        if (ga) {
-            w0 = ll_get(pa);
-            w1 = ll_get(pa + n);
-        }
-        if (gb) {
-            w2 = ll_get(pb);
-            w3 = ll_get(pb + n);
-        }
-        const bool ok = (!ga || (ll_is(w0, tag) && ll_is(w1, tag))) && (!gb || (ll_is(w2, tag) && ll_is(w3, tag)));
-        if (dead || __all(ok)) break;
-        if (t >= p.max_polls) {   // a neighbour that never answers: give up, and tell everyone
-            __hip_atomic_store(p.failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            dead = true;
-        } else if ((t & 1023) == 1023) {
-            dead = __hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-        }
-    }
-    a0 = ll_val(w0);
-    a1 = ll_val(w1);
-    b0 = ll_val(w2);
-    b1 = ll_val(w3);
-}
 
 // A unit is one 64-cell segment of one row of the tile; its six components
 // lie side by side in LDS ([unit][6][64]), so one base address and immediate
@@ -93,32 +48,16 @@ __device__ __forceinline__ void ll_wait(const PArgs &p, bool ga, const u64 *pa, 
 // coefficients, x-slab psi and (up to three units) y- and z-slab psi stay in
 // registers.  What a half-step needs to know about a unit is the same on
 // every lane and every step (PUnit, built by the host, in the order the
-// half-step takes the units: those that wait for a neighbour's row last); a
-// wave holds the 16 words of four units in the lanes of one register.
+// half-step takes the units: those that wait for a neighbour's row last).
 template <int NU>
-struct PDesc {
-    int v[(NU + 3) / 4];
-    __device__ __forceinline__ void load(const PUnit *u, int w, int nu, int lane)
-    {
-        for (int q = 0; q < (NU + 3) / 4; ++q) {
-            const int n = w + (4 * q + lane / 16) * PW;
-            v[q] = n < nu ? ((const int *)(u + n))[lane % 16] : 0;
-        }
-    }
-    __device__ __forceinline__ PUnit at(int n) const
-    {
-        PUnit u;
-        const int r = v[n / 4], l = (n % 4) * 16;
-        u.lds = __builtin_amdgcn_readlane(r, l); u.flags = __builtin_amdgcn_readlane(r, l + 1);
-        u.i0 = __builtin_amdgcn_readlane(r, l + 2); u.j = __builtin_amdgcn_readlane(r, l + 3);
-        u.k = __builtin_amdgcn_readlane(r, l + 4); u.psx = __builtin_amdgcn_readlane(r, l + 5);
-        u.psy = __builtin_amdgcn_readlane(r, l + 6); u.psz = __builtin_amdgcn_readlane(r, l + 7);
-        u.wj = __builtin_amdgcn_readlane(r, l + 8); u.wk = __builtin_amdgcn_readlane(r, l + 9);
-        u.oj = __builtin_amdgcn_readlane(r, l + 10); u.ok = __builtin_amdgcn_readlane(r, l + 11);
-        u.ev = __builtin_amdgcn_readlane(r, l + 12); u.nev = __builtin_amdgcn_readlane(r, l + 13);
-        return u;
-    }
-};
+__device__ __forceinline__ PUnit unit_of(const PDesc<NU> &d, int n)
+{
+    PUnit u;
+    u.lds = d.at(n, 0); u.flags = d.at(n, 1); u.i0 = d.at(n, 2); u.j = d.at(n, 3); u.k = d.at(n, 4);
+    u.psx = d.at(n, 5); u.psy = d.at(n, 6); u.psz = d.at(n, 7); u.wj = d.at(n, 8); u.wk = d.at(n, 9);
+    u.oj = d.at(n, 10); u.ok = d.at(n, 11); u.ev = d.at(n, 12); u.nev = d.at(n, 13);
+    return u;
+}
 
 // psi of a cell's slabs (two values per axis) and the E coefficients of a unit
 struct PPsi {
@@ -177,7 +116,7 @@ __global__ void __launch_bounds__(64 * PW) persist_kernel(const KArgs a, const P
         ex_[n] = hx_[n] = ey_[np] = ez_[np] = hy_[np] = hz_[np] = PPsi{0.f, 0.f};
         if (w + n * PW >= nu) continue;
         {
-            const PUnit u = de.at(n);
+            const PUnit u = unit_of(de, n);
             const int i = u.i0 + lane;
             const i64 c = (i64)u.k * a.plane + (i64)u.j * a.px + i;
             int cl = 0;
@@ -190,7 +129,7 @@ __global__ void __launch_bounds__(64 * PW) persist_kernel(const KArgs a, const P
             if (YZ && (u.flags & PU_YS) && i < nx) psi_ld(ey_[np], a.psi_exy, a.psi_ezy, u.psy + lane);
             if (YZ && (u.flags & PU_ZS) && i < nx) psi_ld(ez_[np], a.psi_exz, a.psi_eyz, u.psz + lane);
         }
-        const PUnit u = dh.at(n);
+        const PUnit u = unit_of(dh, n);
         const int i = u.i0 + lane;
         const i64 c = (i64)u.k * a.plane + (i64)u.j * a.px + i;
         float *o = sf + u.lds + lane;
@@ -459,13 +398,13 @@ __global__ void __launch_bounds__(64 * PW) persist_kernel(const KArgs a, const P
 #pragma unroll
         for (int n = 0; n < NU; ++n) {
             __builtin_amdgcn_sched_barrier(0);   // one unit's registers at a time
-            if (w + n * PW < nu) e_unit(cf[n], ex_[n], ey_[YZ ? n : 0], ez_[YZ ? n : 0], de.at(n), m, tag);
+            if (w + n * PW < nu) e_unit(cf[n], ex_[n], ey_[YZ ? n : 0], ez_[YZ ? n : 0], unit_of(de, n), m, tag);
         }
         __syncthreads();
 #pragma unroll
         for (int n = 0; n < NU; ++n) {
             __builtin_amdgcn_sched_barrier(0);
-            if (w + n * PW < nu) h_unit(hx_[n], hy_[YZ ? n : 0], hz_[YZ ? n : 0], dh.at(n), m, tag);
+            if (w + n * PW < nu) h_unit(hx_[n], hy_[YZ ? n : 0], hz_[YZ ? n : 0], unit_of(dh, n), m, tag);
         }
         __syncthreads();
     }
@@ -479,13 +418,13 @@ __global__ void __launch_bounds__(64 * PW) persist_kernel(const KArgs a, const P
         if (w + n * PW >= nu) continue;
         const int np = YZ ? n : 0;
         {
-            const PUnit u = de.at(n);
+            const PUnit u = unit_of(de, n);
             const bool in = u.i0 + lane < nx;
             if (xs_e(u)) psi_st(ex_[n], a.psi_eyx, a.psi_ezx, sx_of(u));
             if (YZ && (u.flags & PU_YS) && in) psi_st(ey_[np], a.psi_exy, a.psi_ezy, u.psy + lane);
             if (YZ && (u.flags & PU_ZS) && in) psi_st(ez_[np], a.psi_exz, a.psi_eyz, u.psz + lane);
         }
-        const PUnit u = dh.at(n);
+        const PUnit u = unit_of(dh, n);
         const int i = u.i0 + lane;
         if (xs_h(u)) psi_st(hx_[n], a.psi_hyx, a.psi_hzx, sx_of(u));
         if (YZ && (u.flags & PU_YS) && i < nx) psi_st(hy_[np], a.psi_hxy, a.psi_hzy, u.psy + lane);
@@ -550,18 +489,9 @@ static const void *persist_fn(int storage, int units)
     }
 }
 
-// Whether `tiles` workgroups with `lds` bytes each can be resident at once
-// (and the kernel is set up to use them).
 bool persist_fits(int storage, int units, int tiles, size_t lds, int device)
 {
-    const void *fn = persist_fn(storage, units);
-    int coop = 0, cus = 0, per = 0;
-    bool ok = fn && hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess && coop &&
-              hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-              hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
-              hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, 64 * PW, lds) == hipSuccess;
-    if (!ok) (void)hipGetLastError();
-    return ok && per >= 1 && tiles <= cus * per;
+    return coop_fits(persist_fn(storage, units), tiles, lds, device);
 }
 
 hipError_t launch_persist(int storage, const KArgs &a, const PArgs &p, int tiles, size_t lds, hipStream_t s)
