@@ -334,7 +334,7 @@ __global__ void __launch_bounds__(TX * BY)
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
     int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz);
+    tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     const int i = tx * TX + (int)(threadIdx.x & (TX - 1));
     const int j = ty * BY + (int)(threadIdx.x / TX);
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
@@ -453,7 +453,7 @@ __global__ void __launch_bounds__(TX * BY) adj_h_kernel(const KArgs a, const AAr
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
     int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz);
+    tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     const int i = tx * TX + (int)(threadIdx.x & (TX - 1));
     const int j = ty * BY + (int)(threadIdx.x / TX);
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
@@ -632,7 +632,7 @@ struct AECol {
 // index in the box, x fastest), XCD-aware as remap_tile.
 __device__ __forceinline__ void tile_of_list(const KArgs &a, const int *tl, int ntl, int &tx, int &ty, int &tz)
 {
-    const int e = tl[remap_tile(ntl)];
+    const int e = tl[remap_tile(ntl, blockIdx.x)];
     const int bx = a.ib[3] - a.ib[0], by = a.ib[4] - a.ib[1];
     tx = a.ib[0] + e % bx;
     ty = a.ib[1] + (e / bx) % by;
@@ -887,7 +887,7 @@ __global__ void __launch_bounds__(TX * BY)
     __shared__ HQ sq[2][BY][TX];
     int tx, ty, tz;
     if (IN && b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz);
-    else tile_of_region<V>(a, tx, ty, tz);
+    else tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     AECol cc;
     cc.lane = (int)(threadIdx.x & (TX - 1));
     cc.row = (int)(threadIdx.x / TX);
@@ -1174,7 +1174,7 @@ __global__ void __launch_bounds__(TX * BY)
     __shared__ EQ sq[2][BY][TX];
     int tx, ty, tz;
     if (IN && b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz);
-    else tile_of_region<V>(a, tx, ty, tz);
+    else tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     AECol cc;
     cc.lane = (int)(threadIdx.x & (TX - 1));
     cc.row = (int)(threadIdx.x / TX);

@@ -264,8 +264,9 @@ int upload_tables(fdtd_ctx *c);
 // Planes per z-march block.  Many short marches keep every CU's wave slots
 // full through the tail of a launch; each block re-reads one plane of the
 // carried z-neighbour, so a block of `planes` costs 1/planes extra on that
-// stream.  Measured on slab512: the FP32 E sweep is fastest at 4 planes, the
-// FP32 H sweep at 2, the 16-bit pair sweeps at 8 (FDTD_CHUNKS overrides all
+// stream.  Measured: the FP32 sweeps are fastest at 4 planes (us per step, H
+// at 2 / at 4: 203x149x97 magnetic 66.9 / 64.4, 200^3 154 / 145, 320x320x130
+// magnetic 221 / 207), the 16-bit pair sweeps at 8 (FDTD_CHUNKS overrides all
 // three with a number of blocks along z; FDTD_E_PLANES, FDTD_H_PLANES and
 // FDTD_PAIR_PLANES set one sweep's planes per block before the small-grid
 // halving).
@@ -289,14 +290,14 @@ int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_e
 // z-blocks of kchunk planes): along each axis, the run of tiles whose cell
 // range reaches neither a CPML slab nor an outer face (nor the grid's end).
 // The x-edge variant takes the tiles beside the box in x, the general
-// variant the rows and z-blocks outside it: z-edge variants of their own
-// measured slower on 512x512x256 (their launch tails cost more than their
-// leaner code saves).  FDTD_INTERIOR=0, or an axis without interior tiles,
-// leaves the box empty (z range [0, 0)) and every tile to the general
-// variant.  (On 128x128x64 an x-edge launch over the interior rows and
-// z-blocks beside a general one measured slower than the general variant
-// alone: 32.4 against 26.9 ms for 1000 steps; the two half-size launches
-// of a small grid leave CUs idle.)
+// variant the rows and z-blocks outside it.  Where no column of tiles is
+// interior (nx up to two tiles and a slab), the x-edge variant takes every
+// column of the box's rows and z-blocks, from 3 M cells on for 16-bit
+// storage: us per step, general variant alone / so: FP16 256^3 214 / 178,
+// 220x128x128 62 / 59, 150x131x118 47 / 48, block-scaled int16 261 / 223, 77 /
+// 70, 60 / 64; FP32 (64-cell tiles) 112x150x200 74 / 70, 128x128x100 38.5 /
+// 37.7.  FDTD_INTERIOR=0, or a y or z axis without interior tiles, leaves the
+// box empty (z range [0, 0)) and every tile to the general variant.
 // beyond: cells past the tile's high sides that must lie off the slabs too
 // (the fused step evaluates one).
 void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int beyond = 0)
@@ -318,7 +319,10 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
                 lo = std::min(lo, t);
                 hi = t + 1;
             }
-        if (hi <= lo) return;
+        if (hi <= lo) {
+            if (ax > 0 || sweep == 2 || (tile_cols > 64 && (double)in.nx * in.ny * in.nz < 3e6)) return;
+            lo = hi = 0;
+        }
         box[ax] = lo;
         box[ax + 3] = hi;
     }
@@ -751,7 +755,7 @@ int do_finalize(fdtd_ctx *c)
     a.tiles_x = (in.nx + tile_cols() - 1) / tile_cols();
     a.tiles_y = (in.ny + tile_rows() - 1) / tile_rows();
     a.kchunk = choose_chunks(c, a.tiles_x * a.tiles_y, 4, "FDTD_E_PLANES");
-    c->kchunk_h = choose_chunks(c, a.tiles_x * a.tiles_y, 2, "FDTD_H_PLANES");
+    c->kchunk_h = choose_chunks(c, a.tiles_x * a.tiles_y, 4, "FDTD_H_PLANES");
     // 16-bit storage (FP16, BF16, block-scaled int16) sweeps a cell pair per
     // thread (128-cell tile rows); FDTD_PAIR=0 selects the one-cell kernels
     // instead (same stored bits)

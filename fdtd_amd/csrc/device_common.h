@@ -88,10 +88,10 @@ __device__ __forceinline__ int class_of(const void *cls, i64 c)
 // Workgroup -> tile: XCD x (= blockIdx % 8 under round-robin dispatch) gets
 // the contiguous tile range [start_x, start_x + count_x).  With a light-cone
 // sub-range (a.sub), the tiles of that range only.
-__device__ __forceinline__ void tile_of(const KArgs &a, int &tx, int &ty, int &tz)
+__device__ __forceinline__ void tile_of(const KArgs &a, int &tx, int &ty, int &tz, int b)
 {
     if (a.sub[3] > 0) {
-        const int b = blockIdx.x, nt = a.sub[3] * a.sub[4] * a.sub[5];
+        const int nt = a.sub[3] * a.sub[4] * a.sub[5];
         const int q = nt >> 3, r = nt & 7, x = b & 7;
         const int t = x * q + (x < r ? x : r) + (b >> 3);
         tx = a.sub[0] + t % a.sub[3];
@@ -100,7 +100,6 @@ __device__ __forceinline__ void tile_of(const KArgs &a, int &tx, int &ty, int &t
         return;
     }
     const int nt = a.tiles_x * a.tiles_y * ((a.nz + a.kchunk - 1) / a.kchunk);
-    const int b = blockIdx.x;
     const int q = nt >> 3, r = nt & 7, x = b & 7;
     const int t = x * q + (x < r ? x : r) + (b >> 3);
     tx = t % a.tiles_x;
@@ -110,11 +109,10 @@ __device__ __forceinline__ void tile_of(const KArgs &a, int &tx, int &ty, int &t
 
 
 // Workgroup -> tile of the interior box, with the same XCD-aware remap.
-__device__ __forceinline__ void tile_of_box(const KArgs &a, int &tx, int &ty, int &tz)
+__device__ __forceinline__ void tile_of_box(const KArgs &a, int &tx, int &ty, int &tz, int b)
 {
     const int bx = a.ib[3] - a.ib[0], by = a.ib[4] - a.ib[1];
     const int nt = bx * by * (a.ib[5] - a.ib[2]);
-    const int b = blockIdx.x;
     const int q = nt >> 3, r = nt & 7, x = b & 7;
     const int t = x * q + (x < r ? x : r) + (b >> 3);
     tx = a.ib[0] + t % bx;
@@ -123,14 +121,13 @@ __device__ __forceinline__ void tile_of_box(const KArgs &a, int &tx, int &ty, in
 }
 
 // XCD-aware remap of workgroup b over nt tiles (as in tile_of).
-__device__ __forceinline__ int remap_tile(int nt)
+__device__ __forceinline__ int remap_tile(int nt, int b)
 {
-    const int b = blockIdx.x;
     const int q = nt >> 3, r = nt & 7, x = b & 7;
     return x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// Workgroup -> tile of region variant V, computed from the interior box (no
+// Workgroup b of a region -> tile of region variant V, computed from the interior box (no
 // tile lists: the many short workgroups then start without a dependent
 // load).  V_X: tile columns outside [ib0, ib3) of the box's rows and
 // z-blocks.  V_Z (with zsplit): the box's tile columns and rows in every
@@ -139,14 +136,14 @@ __device__ __forceinline__ int remap_tile(int nt)
 // outside [ib1, ib4) of the box's z-blocks; the whole grid (or the light-cone
 // range) when there is no box.
 template <int V>
-__device__ __forceinline__ void tile_of_region(const KArgs &a, int &tx, int &ty, int &tz)
+__device__ __forceinline__ void tile_of_region(const KArgs &a, int &tx, int &ty, int &tz, int b)
 {
     const int *ib = a.ib;
     if (V == V_IN) {
-        tile_of_box(a, tx, ty, tz);
+        tile_of_box(a, tx, ty, tz, b);
     } else if (V == V_X) {
         const int ex = ib[0] + a.tiles_x - ib[3], by = ib[4] - ib[1];
-        const int t = remap_tile(ex * by * (ib[5] - ib[2]));
+        const int t = remap_tile(ex * by * (ib[5] - ib[2]), b);
         const int xe = t % ex;
         tx = xe < ib[0] ? xe : ib[3] + (xe - ib[0]);
         ty = ib[1] + (t / ex) % by;
@@ -154,19 +151,19 @@ __device__ __forceinline__ void tile_of_region(const KArgs &a, int &tx, int &ty,
     } else if (V == V_Z) {
         const int bx = ib[3] - ib[0], by = ib[4] - ib[1], bz = ib[5] - ib[2];
         const int tzs = (a.nz + a.kchunk - 1) / a.kchunk;
-        const int t = remap_tile(bx * by * (tzs - bz));
+        const int t = remap_tile(bx * by * (tzs - bz), b);
         const int ze = t / (bx * by);
         tx = ib[0] + t % bx;
         ty = ib[1] + (t / bx) % by;
         tz = ze < ib[2] ? ze : ib[5] + (ze - ib[2]);
     } else if (ib[5] == ib[2]) {
-        tile_of(a, tx, ty, tz);
+        tile_of(a, tx, ty, tz, b);
     } else {
         const int txy = a.tiles_x * a.tiles_y, tzs = (a.nz + a.kchunk - 1) / a.kchunk;
         const int bx = ib[3] - ib[0], by = ib[4] - ib[1], bz = ib[5] - ib[2], ey = a.tiles_y - by;
         const int per = a.zsplit ? txy - bx * by : txy;   // tiles per z-block outside the box's z range
         const int n1 = per * (tzs - bz);
-        const int t = remap_tile(n1 + a.tiles_x * ey * bz);
+        const int t = remap_tile(n1 + a.tiles_x * ey * bz, b);
         if (t < n1) {
             const int ze = t / per, u = t % per;
             tz = ze < ib[2] ? ze : ib[5] + (ze - ib[2]);

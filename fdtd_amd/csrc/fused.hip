@@ -398,7 +398,7 @@ __attribute__((amdgpu_waves_per_eu(4))) step_kernel(const KArgs a, const int m)
 {
     __shared__ FShare sh;
     int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz);
+    tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     const int lane = (int)(threadIdx.x & (TX - 1));
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / TX));
     const int i0 = tx * TX, j0 = ty * FY;

@@ -22,6 +22,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "cell_sweep.h"
 #include "device_common.h"
 #include "internal.h"
 #include "sweep_common.h"
@@ -54,7 +55,7 @@ __device__ __forceinline__ QW<bq16_t> qw_next<bq16_t>(const QW<bq16_t> &q, const
 #define P_OCC
 #endif
 
-hipError_t launch_half_step_general(bool efield, int storage, int mode, const KArgs &a, int m, hipStream_t s);
+hipError_t launch_half_step(bool efield, int storage, int mode, const KArgs &a, int m, hipStream_t s);
 
 typedef std::uint32_t u32;
 
@@ -397,10 +398,8 @@ __device__ __forceinline__ void ep_update(const EPair<T> &p, const CoefPair &t, 
 }
 
 template <class T, int CM, int V>
-__global__ void __launch_bounds__(TX * BY) P_OCC e_pair_kernel(const KArgs a, const int m)
+__device__ __forceinline__ void e_pair_tile(const KArgs &a, const int m, const int tx, const int ty, const int tz)
 {
-    int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz);
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int i0 = tx * TXP + 2 * (int)(threadIdx.x & (TX - 1));
     PRow r;
@@ -683,10 +682,8 @@ __device__ __forceinline__ void hp_update(const HPair<T> &p, const CoefPair &t, 
 }
 
 template <class T, int CM, int V>
-__global__ void __launch_bounds__(TX * BY) P_OCC h_pair_kernel(const KArgs a, const int m)
+__device__ __forceinline__ void h_pair_tile(const KArgs &a, const int m, const int tx, const int ty, const int tz)
 {
-    int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz);
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int i0 = tx * TXP + 2 * (int)(threadIdx.x & (TX - 1));
     PRow r;
@@ -769,19 +766,70 @@ __global__ void __launch_bounds__(TX * BY) P_OCC h_pair_kernel(const KArgs a, co
     }
 }
 
-// ---- launchers --------------------------------------------------------------
-template <class T, int V>
-static void launch_pair_v(bool efield, int mode, const KArgs &a, int m, int nt, hipStream_t s)
+// A half-step in one launch, as kernels.hip's: the general variant's tiles
+// first, then the x-edge ones, then the interior.  CELLS: the general variant
+// runs one cell per thread, the left halves of its ng 128-cell tiles and then
+// the right ones.  One launch against one for each variant, us per step (FP16):
+// 512x512x256 680 / 656, 300x200x200 163 / 140, 512x200x64 98 / 75; block-
+// scaled int16 808 / 806, 203 / 174, 123 / 95.
+template <class T, int CM, bool CELLS>
+__global__ void __launch_bounds__(TX * BY) P_OCC e_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
-    dim3 grid(nt), block(TX * BY);
-    if (efield) {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((e_pair_kernel<T, CLS_UNIFORM, V>), grid, block, 0, s, a, m);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((e_pair_kernel<T, CLS_U16, V>), grid, block, 0, s, a, m);
-        else hipLaunchKernelGGL((e_pair_kernel<T, CLS_U32, V>), grid, block, 0, s, a, m);
+    const int b = blockIdx.x, n = CELLS ? 2 * ng : ng;
+    int tx, ty, tz;
+    if (b < n) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, b < ng ? b : b - ng);
+        if constexpr (CELLS) {
+            tx = 2 * tx + (b < ng ? 0 : 1);
+            if (tx * TX < a.nx) e_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        } else {
+            e_pair_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        }
+    } else if (b < n + nx) {
+        tile_of_region<V_X>(a, tx, ty, tz, b - n);
+        e_pair_tile<T, CM, V_X>(a, m, tx, ty, tz);
     } else {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((h_pair_kernel<T, CLS_UNIFORM, V>), grid, block, 0, s, a, m);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((h_pair_kernel<T, CLS_U16, V>), grid, block, 0, s, a, m);
-        else hipLaunchKernelGGL((h_pair_kernel<T, CLS_U32, V>), grid, block, 0, s, a, m);
+        tile_of_region<V_IN>(a, tx, ty, tz, b - n - nx);
+        e_pair_tile<T, CM, V_IN>(a, m, tx, ty, tz);
+    }
+}
+template <class T, int CM, bool CELLS>
+__global__ void __launch_bounds__(TX * BY) P_OCC h_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
+{
+    const int b = blockIdx.x, n = CELLS ? 2 * ng : ng;
+    int tx, ty, tz;
+    if (b < n) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, b < ng ? b : b - ng);
+        if constexpr (CELLS) {
+            tx = 2 * tx + (b < ng ? 0 : 1);
+            if (tx * TX < a.nx) h_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        } else {
+            h_pair_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        }
+    } else if (b < n + nx) {
+        tile_of_region<V_X>(a, tx, ty, tz, b - n);
+        h_pair_tile<T, CM, V_X>(a, m, tx, ty, tz);
+    } else {
+        tile_of_region<V_IN>(a, tx, ty, tz, b - n - nx);
+        h_pair_tile<T, CM, V_IN>(a, m, tx, ty, tz);
+    }
+}
+
+// ---- launchers --------------------------------------------------------------
+template <class T, bool CELLS>
+static void launch_pair_all(bool efield, int mode, const KArgs &a, int m, int ng, int nx, int nb, hipStream_t s)
+{
+    dim3 grid(nb + nx + (CELLS ? 2 : 1) * ng), block(TX * BY);
+    if (efield) {
+        if (mode == CLS_UNIFORM)
+            hipLaunchKernelGGL((e_pair_kernel<T, CLS_UNIFORM, CELLS>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((e_pair_kernel<T, CLS_U16, CELLS>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((e_pair_kernel<T, CLS_U32, CELLS>), grid, block, 0, s, a, m, ng, nx);
+    } else {
+        if (mode == CLS_UNIFORM)
+            hipLaunchKernelGGL((h_pair_kernel<T, CLS_UNIFORM, CELLS>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((h_pair_kernel<T, CLS_U16, CELLS>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((h_pair_kernel<T, CLS_U32, CELLS>), grid, block, 0, s, a, m, ng, nx);
     }
 }
 
@@ -790,23 +838,21 @@ static hipError_t launch_pair_t(bool efield, int mode, const KArgs &a, int m, hi
 {
     int nb, nx, nzt, ng;   // nzt = 0: the forward sweeps run without zsplit
     region_tiles(a, nb, nx, nzt, ng);
-    if (nb > 0) launch_pair_v<T, V_IN>(efield, mode, a, m, nb, s);
-    if (nx > 0) launch_pair_v<T, V_X>(efield, mode, a, m, nx, s);
-    if (ng > 0 && !gen_cells) launch_pair_v<T, V_GEN>(efield, mode, a, m, ng, s);
-    if (ng > 0 && gen_cells) {
-        // the same rows and z-blocks in one-cell tiles (TX columns): the
-        // general region depends on the box's y and z range only
+    if (!gen_cells) {
+        launch_pair_all<T, false>(efield, mode, a, m, ng, nx, nb, s);
+    } else if (nb + nx > 0) {
+        launch_pair_all<T, true>(efield, mode, a, m, ng, nx, nb, s);
+    } else {
+        // the general variant alone: the one-cell kernel (the pair kernel's
+        // registers are those of its x-edge variant, too), TX columns a tile
         KArgs c = a;
         c.tiles_x = (a.nx + TX - 1) / TX;
-        c.ib[0] = a.ib[0] * (TXP / TX);
-        c.ib[3] = a.ib[3] * (TXP / TX);
         if (c.sub[3] > 0) {   // light-cone range in one-cell tile columns
             c.sub[0] = a.sub[0] * (TXP / TX);
             c.sub[3] = min(a.sub[3] * (TXP / TX), c.tiles_x - c.sub[0]);
         }
         const int st = std::is_same<T, bf16_t>::value ? 2 : is_bq<T>::value ? 3 : 1;
-        const hipError_t e = launch_half_step_general(efield, st, mode, c, m, s);
-        if (e != hipSuccess) return e;
+        return launch_half_step(efield, st, mode, c, m, s);
     }
     return hipGetLastError();
 }
