@@ -40,6 +40,8 @@ size_t persist_lds(int units, int sx);
 int persist_max_units();
 bool persist_fits(int storage, int units, int tiles, size_t lds, int device);
 hipError_t launch_persist(int storage, const KArgs &a, const PArgs &p, int tiles, size_t lds, hipStream_t s);
+hipError_t launch_unpack(int storage, const void *f, const std::uint8_t *q, float *out, std::uint32_t g0, std::uint32_t n,
+                         int nx, int px, float scale, hipStream_t s);
 size_t adj_persist_lds(int units, int sx, int events);
 int adj_persist_max_units();
 bool adj_persist_fits(int units, int tiles, size_t lds, int device);
@@ -112,6 +114,8 @@ struct fdtd_ctx {
     int adj_segments = 0;
     uint64_t adj_bytes = 0;         // peak device memory of the last adjoint run
     hipEvent_t adj_ev[3] = {};      // timing events of the adjoint (made at create)
+    float *stage = nullptr;         // pinned memory of fdtd_get_field, two pieces of STAGE floats
+    hipEvent_t stage_ev[2] = {};
     unsigned char *scratch = nullptr;   // this device's copy of the static scratch
 };
 
@@ -960,6 +964,8 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
     return e;
 }
 
+constexpr size_t STAGE = 1 << 20;   // floats of a piece of fdtd_get_field
+
 // Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
 // and the call enough steps to pay for it.
 constexpr int P_MIN_STEPS = 4;
@@ -1003,6 +1009,19 @@ int check_advance(fdtd_ctx *c)
     return fail(c, FDTD_E_DEVICE, "a workgroup waited too long for a neighbour's rows; the state is not valid "
                 "(fdtd_reset starts over)");
 }
+
+// The context's device current on this thread, for a scope.
+struct DeviceGuard {
+    int was = -1;
+    explicit DeviceGuard(int device)
+    {
+        if (hipGetDevice(&was) != hipSuccess || was == device || hipSetDevice(device) != hipSuccess) was = -1;
+    }
+    ~DeviceGuard()
+    {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
 
 // A stream of one call, drained and destroyed on every return path.
 struct StreamGuard {
@@ -1637,6 +1656,9 @@ int fdtd_destroy(fdtd_ctx *c)
     free_device(c);
     for (hipEvent_t e : c->adj_ev)
         if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stage) (void)hipHostFree(c->stage);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return FDTD_OK;
@@ -1995,38 +2017,37 @@ int fdtd_get_field(fdtd_ctx *c, int comp, float *out, size_t n)
     const int nx = c->in.nx, ny = c->in.ny, nz = c->in.nz, px = c->in.px;
     const size_t cells = (size_t)nx * ny * nz;
     if (n < cells) return fail(c, FDTD_E_INVALID, "output too small");
-    std::vector<unsigned char> raw((size_t)px * ny * nz * c->esz);
-    const char *base = (const char *)c->fields[comp] + (size_t)c->ka.plane * c->esz;
-    HIPCHK(c, hipMemcpy(raw.data(), base, raw.size(), hipMemcpyDeviceToHost));
-    std::vector<std::uint8_t> qraw;   // the component's exponent array, k = 0 .. nz-1
-    if (c->qarr[comp / 3]) {
-        qraw.resize((size_t)px * ny * nz / BQ_BLOCK * BQ_STRIDE);
-        HIPCHK(c, hipMemcpy(qraw.data(), c->qarr[comp / 3] + (size_t)c->ka.plane / BQ_BLOCK * BQ_STRIDE,
-                            qraw.size(), hipMemcpyDeviceToHost));
-    }
-    const float un = c->built.probe_unscale[comp];
-    for (size_t r = 0; r < (size_t)ny * nz; ++r)
-        for (int i = 0; i < nx; ++i) {
-            const size_t src = r * px + i;
-            float v;
-            if (c->esz == 4) {
-                std::memcpy(&v, &raw[src * 4], 4);
-            } else {
-                uint16_t h;
-                std::memcpy(&h, &raw[src * 2], 2);
-                if (c->in.storage == FDTD_STORE_BF16) {
-                    uint32_t u = (uint32_t)h << 16;
-                    std::memcpy(&v, &u, 4);
-                } else if (c->in.storage == FDTD_STORE_BQ16) {
-                    v = std::ldexp((float)(int16_t)h, (int)qraw[src / BQ_BLOCK * BQ_STRIDE + comp % 3] - BQ_BIAS);
-                } else {
-                    _Float16 f;
-                    std::memcpy(&f, &h, 2);
-                    v = (float)f;
-                }
-            }
-            out[r * nx + i] = v * un;
+    DeviceGuard dg(c->device);
+    // two pieces of pinned memory, made at the first call and kept: the GPU
+    // packs and converts one while the other is copied out.  Through a copy of
+    // the padded array in pageable memory and a loop here, the six fields of
+    // 150x131x118 took 14.5 ms; so 6.3, most of it the copy out (9 GB/s).
+    if (!c->stage) {
+        for (auto &e : c->stage_ev)
+            if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        if (hipHostMalloc((void **)&c->stage, 2 * STAGE * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->stage = nullptr;
+            return fail(c, FDTD_E_NOMEM, "pinned host memory (%zu bytes)", 2 * STAGE * sizeof(float));
         }
+    }
+    const char *base = (const char *)c->fields[comp] + (size_t)c->ka.plane * c->esz;
+    const std::uint8_t *qe = c->qexp[comp] ? c->qexp[comp] + (size_t)c->ka.plane / BQ_BLOCK * BQ_STRIDE : nullptr;
+    const float un = c->built.probe_unscale[comp];
+    const size_t pieces = (cells + STAGE - 1) / STAGE;
+    for (size_t p = 0; p <= pieces; ++p) {
+        if (p < pieces) {
+            const size_t g = p * STAGE, len = std::min(STAGE, cells - g);
+            HIPCHK(c, launch_unpack(c->in.storage, base, qe, c->stage + p % 2 * STAGE, (std::uint32_t)g,
+                                    (std::uint32_t)len, nx, px, un, c->stream));
+            HIPCHK(c, hipEventRecord(c->stage_ev[p % 2], c->stream));
+        }
+        if (p > 0) {
+            const size_t g = (p - 1) * STAGE, len = std::min(STAGE, cells - g);
+            HIPCHK(c, hipEventSynchronize(c->stage_ev[(p - 1) % 2]));
+            std::memcpy(out + g, c->stage + (p - 1) % 2 * STAGE, len * sizeof(float));
+        }
+    }
     return FDTD_OK;
 }
 

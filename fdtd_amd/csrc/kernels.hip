@@ -96,6 +96,41 @@ hipError_t launch_half_step(bool efield, int storage, int mode, const KArgs &a, 
     }
 }
 
+// Values g0 .. g0 + n - 1 of a component ([nz][ny][nx], SI) to `out`, pinned
+// host memory: rows packed, converted and scaled on the way, one 4-byte store
+// a lane.  f, q: the component and (block-scaled) its exponents at plane 0.
+// Bound by the link to the host (50 GB/s).
+template <class T>
+__global__ void __launch_bounds__(256)
+    unpack_kernel(const T *f, const std::uint8_t *q, float *out, std::uint32_t g0, std::uint32_t n, std::uint32_t nx,
+                  std::uint32_t px, float scale)
+{
+    const std::uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= n) return;
+    const std::uint32_t r = (g0 + e) / nx, i = (g0 + e) % nx;
+    const i64 c = (i64)r * px + i;
+    float v;
+    if constexpr (is_bq<T>::value) v = ldexpf((float)f[c].v, (int)q[c / BQ_BLOCK * BQ_STRIDE] - BQ_BIAS);
+    else v = ld(f + c);
+    out[e] = v * scale;
+}
+
+hipError_t launch_unpack(int storage, const void *f, const std::uint8_t *q, float *out, std::uint32_t g0, std::uint32_t n,
+                         int nx, int px, float scale, hipStream_t s)
+{
+    dim3 grid((n + 255) / 256), block(256);
+    switch (storage) {
+    case 0: hipLaunchKernelGGL((unpack_kernel<float>), grid, block, 0, s, (const float *)f, q, out, g0, n, nx, px, scale); break;
+    case 1:
+        hipLaunchKernelGGL((unpack_kernel<_Float16>), grid, block, 0, s, (const _Float16 *)f, q, out, g0, n, nx, px, scale);
+        break;
+    case 2: hipLaunchKernelGGL((unpack_kernel<bf16_t>), grid, block, 0, s, (const bf16_t *)f, q, out, g0, n, nx, px, scale); break;
+    case 3: hipLaunchKernelGGL((unpack_kernel<bq16_t>), grid, block, 0, s, (const bq16_t *)f, q, out, g0, n, nx, px, scale); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 int tile_rows() { return BY; }
 int tile_cols() { return TX; }
 
