@@ -336,14 +336,16 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
 // The fused step's tiling and its second buffers; without the memory for
 // them the context steps with the two sweeps.
 //
-// The rule: FP32 grids of 14 M cells or more whose interior tiles hold 3/8 of
-// the cells (half of them where the H coefficients differ by cell, which costs
-// the fused kernel 16 registers).  The fused pass gains on interior tiles;
-// its general variant, with both half-steps' slab state, does not, and its
-// workgroups are fewer and longer.  Measured, us per step, sweeps / fused:
-// 512x512x256 1086 / 947, 256^3 292 / 281, 320x320x160 292 / 277, magnetic
-// 512x512x128 593 / 574; below the line 224^3 213 / 224, 512x512x64 303 / 314
-// (interior a third), magnetic 256^3 302 / 332, 128x128x64 27 / 36.
+// The rule: FP32 grids of 24 M cells or more (60 M where the H coefficients
+// differ by cell, which costs the fused kernel 16 registers) whose interior
+// tiles hold 3/8 of the cells (half).  The fused pass gains on interior tiles
+// and where the fields are read from HBM; its general variant, with both
+// half-steps' slab state, does not, and its workgroups are fewer and longer.
+// Measured, us per step, sweeps / fused: 512x512x256 1061 / 937, 384x384x200
+// 488 / 446, 448x256x256 468 / 430, 300^3 463 / 448; below the line 288^3 400
+// / 409, 512x300x150 380 / 363, 260x260x300 376 / 398, 320x320x160 254 / 271,
+// 256^3 262 / 277.  Magnetic 512x512x256 1094 / 1081, 640x400x256 1055 / 993;
+// below 512x512x200 900 / 922, 512x512x128 573 / 634, 256^3 280 / 328.
 // FDTD_FUSED=0 / 1 overrides it.  Blocks of 16 planes, halved until a launch
 // has 4096 workgroups (256^3: 8 planes 281 us, 16 planes 296).
 void setup_fused(fdtd_ctx *c)
@@ -359,7 +361,8 @@ void setup_fused(fdtd_ctx *c)
     const int *ib = c->box[2];
     const double cells = (double)in.nx * in.ny * in.nz;
     const double inner = (double)(ib[3] - ib[0]) * tile_cols() * (ib[4] - ib[1]) * by * (ib[5] - ib[2]) * c->kchunk_f;
-    if (!force && (cells < 14e6 || inner < (c->h_mode == CLS_UNIFORM ? 0.375 : 0.5) * cells)) return;
+    const bool uni = c->h_mode == CLS_UNIFORM;
+    if (!force && (cells < (uni ? 24e6 : 60e6) || inner < (uni ? 0.375 : 0.5) * cells)) return;
 
     const size_t n_allocs = c->allocs.size();
     const uint64_t bytes = c->dev_bytes;
