@@ -328,13 +328,11 @@ bool adj_stores_quantities(int nx)
 // fstep >= 0: finalize the E half-step of forward step fstep first.
 // sten: gather the transposed H half-step of step m and inject dJ/ds[m].
 template <int CM, int V>
-__global__ void __launch_bounds__(TX * BY)
-    adj_e_kernel(const KArgs a, const AArgs b, const int m, const int fstep, const int sten, const int euni)
+__device__ __forceinline__ void adj_e_tile(const KArgs &a, const AArgs &b, const int m, const int fstep, const int sten,
+                                           const int euni, const int tx, const int ty, const int tz)
 {
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
-    int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     const int i = tx * TX + (int)(threadIdx.x & (TX - 1));
     const int j = ty * BY + (int)(threadIdx.x / TX);
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
@@ -448,12 +446,11 @@ __global__ void __launch_bounds__(TX * BY)
 }
 
 template <int CM, int V>
-__global__ void __launch_bounds__(TX * BY) adj_h_kernel(const KArgs a, const AArgs b, const int euni, const int huni)
+__device__ __forceinline__ void adj_h_tile(const KArgs &a, const AArgs &b, const int euni, const int huni, const int tx,
+                                           const int ty, const int tz)
 {
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
-    int tx, ty, tz;
-    tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     const int i = tx * TX + (int)(threadIdx.x & (TX - 1));
     const int j = ty * BY + (int)(threadIdx.x / TX);
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
@@ -630,9 +627,9 @@ struct AECol {
 
 // Interior tile of a workgroup from a list of tiles of the box (each its
 // index in the box, x fastest), XCD-aware as remap_tile.
-__device__ __forceinline__ void tile_of_list(const KArgs &a, const int *tl, int ntl, int &tx, int &ty, int &tz)
+__device__ __forceinline__ void tile_of_list(const KArgs &a, const int *tl, int ntl, int &tx, int &ty, int &tz, int b)
 {
-    const int e = tl[remap_tile(ntl, blockIdx.x)];
+    const int e = tl[remap_tile(ntl, b)];
     const int bx = a.ib[3] - a.ib[0], by = a.ib[4] - a.ib[1];
     tx = a.ib[0] + e % bx;
     ty = a.ib[1] + (e / bx) % by;
@@ -878,16 +875,12 @@ __device__ __forceinline__ void ae_update(const KArgs &a, const AArgs &b, const 
 // fstep >= 0: finalize the E half-step of forward step fstep first.
 // sten: gather the transposed H half-step of step m and inject dJ/ds[m].
 template <int CM, int V>
-__global__ void __launch_bounds__(TX * BY)
-    adj_e_lds_kernel(const KArgs a, const AArgs b, const int m, const int fstep, const int sten, const int euni,
-                     const int huni)
+__device__ __forceinline__ void adj_e_lds_tile(const KArgs &a, const AArgs &b, const int m, const int fstep,
+                                               const int sten, const int euni, const int huni, HQ (*sq)[BY][TX],
+                                               const int tx, const int ty, const int tz)
 {
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
-    __shared__ HQ sq[2][BY][TX];
-    int tx, ty, tz;
-    if (IN && b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz);
-    else tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     AECol cc;
     cc.lane = (int)(threadIdx.x & (TX - 1));
     cc.row = (int)(threadIdx.x / TX);
@@ -1166,15 +1159,11 @@ __device__ __forceinline__ void ah_update(const KArgs &a, const AArgs &b, const 
 }
 
 template <int CM, int V>
-__global__ void __launch_bounds__(TX * BY)
-    adj_h_lds_kernel(const KArgs a, const AArgs b, const int euni, const int huni)
+__device__ __forceinline__ void adj_h_lds_tile(const KArgs &a, const AArgs &b, const int euni, const int huni,
+                                               EQ (*sq)[BY][TX], const int tx, const int ty, const int tz)
 {
     constexpr bool IN = V == V_IN;   // interior tiles: no slab, face or range predicates
     constexpr bool PX = (V & V_X) != 0, PY = (V & V_Y) != 0, PZ = (V & V_Z) != 0;   // predicated axes
-    __shared__ EQ sq[2][BY][TX];
-    int tx, ty, tz;
-    if (IN && b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz);
-    else tile_of_region<V>(a, tx, ty, tz, blockIdx.x);
     AECol cc;
     cc.lane = (int)(threadIdx.x & (TX - 1));
     cc.row = (int)(threadIdx.x / TX);
@@ -1458,10 +1447,9 @@ __device__ __forceinline__ void fz_step(const FPlane &p, const Tab3 &hu, const f
 }
 
 template <int CM>
-__global__ void __launch_bounds__(TX * BY) adj_fused_kernel(const KArgs a, const AArgs b, const int fin, const int euni)
+__device__ __forceinline__ void adj_fused_tile(const KArgs &a, const AArgs &b, const int fin, const int euni,
+                                               const int tx, const int ty, const int tz)
 {
-    int tx, ty, tz;
-    tile_of_list(a, b.fl, b.nfl, tx, ty, tz);
     const int lane = (int)(threadIdx.x & (TX - 1)), row = (int)(threadIdx.x / TX);
     const int i = tx * TX + lane, j = ty * BY + row;
     const int k0 = tz * a.kchunk, k1 = min(a.nz, k0 + a.kchunk);   // box z-blocks end below the top slab
@@ -1501,11 +1489,105 @@ __global__ void __launch_bounds__(TX * BY) adj_fused_kernel(const KArgs a, const
     if (kk == k1) fz_step(B, hu, a.etab, fn, c, en, hn, o0 + (u32)kk * ob, ob, false, true);
 }
 
+// A reverse half-step in one launch: the general variant's workgroups first
+// (they take longest), then the x-edge, z-slab (wide grids) and interior ones,
+// and in the E sweep the fused interior pass, which touches other cells than
+// the rest of it.  In a launch each the variants leave most of the chip idle
+// at their ends.  Reverse step, us, a launch each (the fused pass on a stream of
+// its own) / so: 576x160x128 453 / 395, 640x150x140 428 / 387, 500x100x80
+// (stored quantities) 221 / 164, 250x120x120 191 / 157, 180x150x100 115 / 86.
+// The wide E sweep's registers are held to four waves per SIMD (133 else).
+struct RegionCounts {
+    int gen, x, z, in, fused;
+};
+template <int CM>
+__global__ void __launch_bounds__(TX * BY)
+    adj_e_kernel(const KArgs a, const AArgs b, const int m, const int fstep, const int sten, const int euni,
+                 const RegionCounts n)
+{
+    int w = blockIdx.x, tx, ty, tz;
+    if (w < n.gen) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, w);
+        adj_e_tile<CM, V_GEN>(a, b, m, fstep, sten, euni, tx, ty, tz);
+    } else if ((w -= n.gen) < n.x) {
+        tile_of_region<V_X>(a, tx, ty, tz, w);
+        adj_e_tile<CM, V_X>(a, b, m, fstep, sten, euni, tx, ty, tz);
+    } else {
+        tile_of_region<V_IN>(a, tx, ty, tz, w - n.x);
+        adj_e_tile<CM, V_IN>(a, b, m, fstep, sten, euni, tx, ty, tz);
+    }
+}
+template <int CM>
+__global__ void __launch_bounds__(TX * BY)
+    adj_h_kernel(const KArgs a, const AArgs b, const int euni, const int huni, const RegionCounts n)
+{
+    int w = blockIdx.x, tx, ty, tz;
+    if (w < n.gen) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, w);
+        adj_h_tile<CM, V_GEN>(a, b, euni, huni, tx, ty, tz);
+    } else if ((w -= n.gen) < n.x) {
+        tile_of_region<V_X>(a, tx, ty, tz, w);
+        adj_h_tile<CM, V_X>(a, b, euni, huni, tx, ty, tz);
+    } else {
+        tile_of_region<V_IN>(a, tx, ty, tz, w - n.x);
+        adj_h_tile<CM, V_IN>(a, b, euni, huni, tx, ty, tz);
+    }
+}
+template <int CM>
+__global__ void __launch_bounds__(TX * BY) __attribute__((amdgpu_waves_per_eu(4)))
+    adj_e_lds_kernel(const KArgs a, const AArgs b, const int m, const int fstep, const int sten, const int euni,
+                     const int huni, const RegionCounts n)
+{
+    __shared__ HQ sq[2][BY][TX];
+    int w = blockIdx.x, tx, ty, tz;
+    if (w < n.gen) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, w);
+        adj_e_lds_tile<CM, V_GEN>(a, b, m, fstep, sten, euni, huni, sq, tx, ty, tz);
+    } else if ((w -= n.gen) < n.x) {
+        tile_of_region<V_X>(a, tx, ty, tz, w);
+        adj_e_lds_tile<CM, V_X>(a, b, m, fstep, sten, euni, huni, sq, tx, ty, tz);
+    } else if ((w -= n.x) < n.z) {
+        tile_of_region<V_Z>(a, tx, ty, tz, w);
+        adj_e_lds_tile<CM, V_Z>(a, b, m, fstep, sten, euni, huni, sq, tx, ty, tz);
+    } else if ((w -= n.z) < n.in) {
+        if (b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz, w);
+        else tile_of_region<V_IN>(a, tx, ty, tz, w);
+        adj_e_lds_tile<CM, V_IN>(a, b, m, fstep, sten, euni, huni, sq, tx, ty, tz);
+    } else {
+        tile_of_list(a, b.fl, b.nfl, tx, ty, tz, w - n.in);
+        adj_fused_tile<CM>(a, b, fstep >= 0, euni, tx, ty, tz);
+    }
+}
+template <int CM>
+__global__ void __launch_bounds__(TX * BY)
+    adj_h_lds_kernel(const KArgs a, const AArgs b, const int euni, const int huni, const RegionCounts n)
+{
+    __shared__ EQ sq[2][BY][TX];
+    int w = blockIdx.x, tx, ty, tz;
+    if (w < n.gen) {
+        tile_of_region<V_GEN>(a, tx, ty, tz, w);
+        adj_h_lds_tile<CM, V_GEN>(a, b, euni, huni, sq, tx, ty, tz);
+    } else if ((w -= n.gen) < n.x) {
+        tile_of_region<V_X>(a, tx, ty, tz, w);
+        adj_h_lds_tile<CM, V_X>(a, b, euni, huni, sq, tx, ty, tz);
+    } else if ((w -= n.x) < n.z) {
+        tile_of_region<V_Z>(a, tx, ty, tz, w);
+        adj_h_lds_tile<CM, V_Z>(a, b, euni, huni, sq, tx, ty, tz);
+    } else {
+        w -= n.z;
+        if (b.ntl > 0) tile_of_list(a, b.tl, b.ntl, tx, ty, tz, w);
+        else tile_of_region<V_IN>(a, tx, ty, tz, w);
+        adj_h_lds_tile<CM, V_IN>(a, b, euni, huni, sq, tx, ty, tz);
+    }
+}
+
 // Interior tile box of the adjoint tiling (tiles tcols wide, rows BY, z-blocks
 // of a.kchunk planes): the own cells of a tile and the neighbour quantities it
 // evaluates (one cell beyond it on each side: the E gather reads H at i-1,
 // j-1, k-1, the H gather E at i+1, j+1, k+1) all lie off the CPML slabs and
-// the outer faces.  All zero when an axis has no such tile.
+// the outer faces.  No tile columns when none is such (the x-edge variant takes
+// them all then: reverse step of 128x128x100 61.8 us with the general variant,
+// 56.7 so); all zero when the y or the z axis has no such tile.
 void adj_box(const KArgs &a, int tcols, int ib[6])
 {
     const int n[3] = {a.nx, a.ny, a.nz}, w[3] = {tcols, BY, a.kchunk};
@@ -1521,7 +1603,10 @@ void adj_box(const KArgs &a, int tcols, int ib[6])
                 lo = lo < t ? lo : t;
                 hi = t + 1;
             }
-        if (hi <= lo) return;
+        if (hi <= lo) {
+            if (ax > 0) return;
+            lo = hi = 0;
+        }
         box[ax] = lo;
         box[ax + 3] = hi;
     }
@@ -1570,80 +1655,49 @@ void adj_fuse_tiles(const KArgs &a0, const std::vector<int> &e_first, const std:
     }
 }
 
-// which: 0 adjoint E sweep, 1 adjoint H sweep, 2 the fused interior pass.  a0.ib[0] < 0 asks for the
-// general variant alone (no interior split).
-hipError_t launch_adj(int which, int mode, int euni, int huni, const KArgs &a0, const AArgs &b, int m, int fstep,
+// A reverse half-step: E (efield; with the fused interior pass where b.nfl >
+// 0) or H.  a0.ib[0] < 0 asks for the general variant alone (no interior
+// split).  The fused pass takes the tiles of b.fl, the interior variants the
+// others (b.tl); an E-only pass (sten 0) covers the whole box.
+hipError_t launch_adj(bool efield, int mode, int euni, int huni, const KArgs &a0, const AArgs &b, int m, int fstep,
                       int sten, hipStream_t s)
 {
     const bool stored = adj_stores_quantities(a0.nx);
-    const int tcols = TX;
     KArgs a = a0;
-    a.tiles_x = (a.nx + tcols - 1) / tcols;
+    a.tiles_x = (a.nx + TX - 1) / TX;
     if (a0.ib[0] < 0) {
         for (int q = 0; q < 6; ++q) a.ib[q] = 0;
     } else {
-        adj_box(a, tcols, a.ib);
+        adj_box(a, TX, a.ib);
     }
     // wide grids: the z-slab blocks of the box's columns and rows get a
     // variant with the z predicates only (the general variant costs 2.7x
     // the interior's time per cell there)
     a.zsplit = stored ? 0 : 1;
     a.sub[3] = 0;
-    int n_in, n_x, n_z, n_gen;
-    region_tiles(a, n_in, n_x, n_z, n_gen);
-#define ADJ_E(CMV, V, NT, EU, HU)                                                                                \
-    do {                                                                                                         \
-        if (stored)                                                                                              \
-            hipLaunchKernelGGL((adj_e_kernel<CMV, V>), dim3(NT), dim3(TX * BY), 0, s, a, bb, m, fstep, sten, EU); \
-        else                                                                                                     \
-            hipLaunchKernelGGL((adj_e_lds_kernel<CMV, V>), dim3(NT), dim3(TX * BY), 0, s, a, bb, m, fstep, sten, \
-                               EU, HU);                                                                          \
-    } while (0)
-#define ADJ_H(CMV, V, NT, EU, HU)                                                                            \
-    do {                                                                                                     \
-        if (stored) hipLaunchKernelGGL((adj_h_kernel<CMV, V>), dim3(NT), dim3(TX * BY), 0, s, a, bb, EU, HU); \
-        else hipLaunchKernelGGL((adj_h_lds_kernel<CMV, V>), dim3(NT), dim3(TX * BY), 0, s, a, bb, EU, HU);    \
-    } while (0)
-#define ADJ_V(MAC, V, NT)                                    \
-    do {                                                     \
-        if (mode == CLS_U32) MAC(CLS_U32, V, NT, euni, huni); \
-        else if (mode == CLS_U16) MAC(CLS_U16, V, NT, euni, huni); \
-        else MAC(CLS_UNIFORM, V, NT, 1, 1);                  \
-    } while (0)
-    // fused interior sweep (b.nfl > 0, which 2): the interior E and H sweeps
-    // take the other tiles (b.tl).  The caller runs it after the previous
-    // step's H sweep and before this step's, beside or after this step's E
-    // sweep (they touch different cells).  An E-only pass (sten 0) covers the
-    // whole box.
+    RegionCounts n{};
+    region_tiles(a, n.in, n.x, n.z, n.gen);
     const bool fuse = !stored && b.nfl > 0 && sten;
     AArgs bb = b;
     if (!fuse) bb.ntl = 0;
-    if (fuse && n_in) n_in = b.ntl;
-    if (which == 2) {
-        if (fuse) {
-            const int nt = b.nfl, fin = fstep >= 0 ? 1 : 0;
-            if (mode == CLS_U32)
-                hipLaunchKernelGGL((adj_fused_kernel<CLS_U32>), dim3(nt), dim3(TX * BY), 0, s, a, b, fin, euni);
-            else if (mode == CLS_U16)
-                hipLaunchKernelGGL((adj_fused_kernel<CLS_U16>), dim3(nt), dim3(TX * BY), 0, s, a, b, fin, euni);
-            else hipLaunchKernelGGL((adj_fused_kernel<CLS_UNIFORM>), dim3(nt), dim3(TX * BY), 0, s, a, b, fin, 1);
-        }
-        return hipGetLastError();
-    }
-    if (which == 0) {
-        if (n_in) ADJ_V(ADJ_E, V_IN, n_in);
-        if (n_x) ADJ_V(ADJ_E, V_X, n_x);
-        if (n_z) ADJ_V(ADJ_E, V_Z, n_z);
-        if (n_gen) ADJ_V(ADJ_E, V_GEN, n_gen);
-    } else {
-        if (n_in) ADJ_V(ADJ_H, V_IN, n_in);
-        if (n_x) ADJ_V(ADJ_H, V_X, n_x);
-        if (n_z) ADJ_V(ADJ_H, V_Z, n_z);
-        if (n_gen) ADJ_V(ADJ_H, V_GEN, n_gen);
-    }
-#undef ADJ_V
-#undef ADJ_E
-#undef ADJ_H
+    if (fuse && n.in) n.in = b.ntl;
+    if (fuse && efield) n.fused = b.nfl;
+    if (mode == CLS_UNIFORM) euni = huni = 1;
+    const dim3 grid(n.gen + n.x + n.z + n.in + n.fused), block(TX * BY);
+    if (grid.x == 0) return hipSuccess;
+#define ADJ(CM)                                                                                               \
+    do {                                                                                                      \
+        if (stored && efield)                                                                                 \
+            hipLaunchKernelGGL((adj_e_kernel<CM>), grid, block, 0, s, a, bb, m, fstep, sten, euni, n);        \
+        else if (stored) hipLaunchKernelGGL((adj_h_kernel<CM>), grid, block, 0, s, a, bb, euni, huni, n);     \
+        else if (efield)                                                                                      \
+            hipLaunchKernelGGL((adj_e_lds_kernel<CM>), grid, block, 0, s, a, bb, m, fstep, sten, euni, huni, n); \
+        else hipLaunchKernelGGL((adj_h_lds_kernel<CM>), grid, block, 0, s, a, bb, euni, huni, n);             \
+    } while (0)
+    if (mode == CLS_U32) ADJ(CLS_U32);
+    else if (mode == CLS_U16) ADJ(CLS_U16);
+    else ADJ(CLS_UNIFORM);
+#undef ADJ
     return hipGetLastError();
 }
 
