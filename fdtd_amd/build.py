@@ -14,7 +14,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libfdtd_amd.so")
-SOURCES = ["api.hip", "kernels.hip", "kernels_pair.hip", "fused.hip", "persist.hip", "adjoint.hip", "adj_persist.hip",
+SOURCES = ["api.hip", "kernels.hip", "kernels_pair.hip", "kernels_f16.hip", "kernels_bf16.hip",
+           "kernels_bq16.hip", "fused.hip", "persist.hip", "adjoint.hip", "adj_persist.hip",
            "scene.cpp", "port.cpp", "marching_loop.cpp"]
 
 HIPCC_FLAGS = [

@@ -819,6 +819,20 @@ int do_finalize(fdtd_ctx *c)
         int rc = dev_alloc(c, &c->psi[p], std::max<size_t>(c->psi_elems[p], 1) * c->esz);
         if (rc) return rc;
     }
+    // The half-steps go past the caches with the swept field's own values
+    // (V_STREAM) once the state -- fields, psi, class map -- is larger than
+    // 300 MB: below that most of it stays in the 256 MB Infinity Cache for the
+    // next half-step.  us per step, past the caches / through them: FP32 150^3
+    // (128 MB) 71 / 54, 190^3 (217) 107 / 88, 200^3 (320: rows of 256) 144 /
+    // 153, 224^3 191 / 205; FP16 230^3 147 / 119, 256^3 (268) 177 / 161,
+    // 512x512x64 (325) 198 / 201, 270^3 (370) 242 / 256; block-scaled int16
+    // 256^3 (284) 220 / 209, 270^3 307 / 320.  FDTD_STREAM=0 / 1 overrides it.
+    {
+        size_t bytes = 6 * (size_t)c->field_elems * c->esz + 2 * c->qarr_bytes + (b.mode == CLS_UNIFORM ? 0 : cls_bytes);
+        for (int p = 0; p < 12; ++p) bytes += c->psi_elems[p] * c->esz;
+        const char *sv = std::getenv("FDTD_STREAM");
+        a.stream = sv ? std::atoi(sv) != 0 : bytes > 300000000;
+    }
     a.e_uni = b.e_uniform ? 1 : 0;
     a.h_uni = b.h_uniform ? 1 : 0;
     int rc;

@@ -94,9 +94,9 @@ __device__ __forceinline__ void e_fetch(EPlane &p, const KArgs &a, const ECol &c
     p.hz_im = fldw(hz, oim, wim, 2);
     p.hx_jm = fldw(hx, ojm, wjm, 0);
     p.hz_jm = fldw(hz, ojm, wjm, 2);
-    p.ex0 = fldnw(ex, o, we, 0);
-    p.ey0 = fldnw(ey, o, we, 1);
-    p.ez0 = fldnw(ez, o, we, 2);
+    p.ex0 = fldnw<(V & V_STREAM) != 0>(ex, o, we, 0);
+    p.ey0 = fldnw<(V & V_STREAM) != 0>(ey, o, we, 1);
+    p.ez0 = fldnw<(V & V_STREAM) != 0>(ez, o, we, 2);
     // class map (no guard planes): the entry of plane k+1
     p.cln = (CM != CLS_UNIFORM && k + 1 < k1)
                 ? class_at<CM>(a.cls, (std::uint32_t)(k + 1) * (std::uint32_t)a.plane + (std::uint32_t)cc.col)
@@ -210,9 +210,9 @@ __device__ __forceinline__ void e_update(const EPlane &p, const Coef &t, const K
         if (cc.jlo) exn = exn + (cx.z * dz) * pex;
         if (cc.ilo) eyn = eyn + (cy.y * dz) * pey;
     }
-    const std::uint32_t bx = fst(ex, o, upd_x, exn, ex0, cc.valid);
-    const std::uint32_t by = fst(ey, o, upd_y, eyn, ey0, cc.valid);
-    const std::uint32_t bz = fst(ez, o, upd_z, ezn, ez0, cc.valid);
+    const std::uint32_t bx = fst<(V & V_STREAM) != 0>(ex, o, upd_x, exn, ex0, cc.valid);
+    const std::uint32_t by = fst<(V & V_STREAM) != 0>(ey, o, upd_y, eyn, ey0, cc.valid);
+    const std::uint32_t bz = fst<(V & V_STREAM) != 0>(ez, o, upd_z, ezn, ez0, cc.valid);
     stq<T>(qp.ex, o, bx, by, bz, cc.valid && (cc.i & (BQ_BLOCK - 1)) == 0);
     if (cc.in_snap && k >= a.sb[2] && k < a.sb[2] + a.sb[5])   // stored-precision value, as the next step reads it
         e_snapshot(ra, cc.i, cc.j, k, m, upd_x ? rnd(exn, ex) : ex0, upd_y ? rnd(eyn, ex) : ey0,
@@ -355,9 +355,9 @@ __device__ __forceinline__ void h_fetch(HPlane &p, const KArgs &a, const HCol &c
     p.ey_ip = fldw(ey, oip, wip, 1);
     p.ez_jp = fldw(ez, ojp, wjp, 2);
     p.ex_jp = fldw(ex, ojp, wjp, 0);
-    p.hx0 = fldnw(hx, o, wh, 0);
-    p.hy0 = fldnw(hy, o, wh, 1);
-    p.hz0 = fldnw(hz, o, wh, 2);
+    p.hx0 = fldnw<(V & V_STREAM) != 0>(hx, o, wh, 0);
+    p.hy0 = fldnw<(V & V_STREAM) != 0>(hy, o, wh, 1);
+    p.hz0 = fldnw<(V & V_STREAM) != 0>(hz, o, wh, 2);
     p.cln = (CM != CLS_UNIFORM && k + 1 < k1)
                 ? class_at<CM>(a.cls, (std::uint32_t)(k + 1) * (std::uint32_t)a.plane + (std::uint32_t)cc.col)
                 : 0;
@@ -458,9 +458,9 @@ __device__ __forceinline__ void h_update(const HPlane &p, const Coef &t, const K
         if (cc.jhi) hxn = hxn + (cx.y * dz) * phx;
         if (cc.ihi) hyn = hyn + (cy.z * dz) * phy;
     }
-    const std::uint32_t bx = fst(hx, o, upd_x, hxn, hx0, cc.valid);
-    const std::uint32_t by = fst(hy, o, upd_y, hyn, hy0, cc.valid);
-    const std::uint32_t bz = fst(hz, o, upd_z, hzn, hz0, cc.valid);
+    const std::uint32_t bx = fst<(V & V_STREAM) != 0>(hx, o, upd_x, hxn, hx0, cc.valid);
+    const std::uint32_t by = fst<(V & V_STREAM) != 0>(hy, o, upd_y, hyn, hy0, cc.valid);
+    const std::uint32_t bz = fst<(V & V_STREAM) != 0>(hz, o, upd_z, hzn, hz0, cc.valid);
     stq<T>(qp.hx, o, bx, by, bz, cc.valid && (cc.i & (BQ_BLOCK - 1)) == 0);
     ex_c = carry(ex_kp);
     ey_c = carry(ey_kp);

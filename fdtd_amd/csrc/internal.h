@@ -39,7 +39,9 @@ struct SrcEdge {
 
 // Sweep-kernel region variants: bit V_X / V_Y / V_Z set when the tiles of
 // the variant can meet an x / y / z CPML slab or outer face.
-enum SweepRegion { V_IN = 0, V_X = 1, V_Y = 2, V_Z = 4, V_GEN = 7 };
+// The forward half-steps' variants have V_STREAM where the swept field's own
+// values are read and written past the caches.
+enum SweepRegion { V_IN = 0, V_X = 1, V_Y = 2, V_Z = 4, V_GEN = 7, V_STREAM = 8 };
 
 // Kernel argument block.  Field pointers point at (i,j,k) = (0,0,0) of an
 // allocation that has one zero guard plane below k = 0 and one above
@@ -91,6 +93,7 @@ struct KArgs {
     // each sweep's tiling when the step is launched (no interior box then).
     int lc[6];
     int sub[6];
+    int stream;                // half-steps with V_STREAM
     int rec;                   // record probes / DFT (0 during adjoint recompute)
     int e_uni, h_uni;          // E / H coefficients are one class (no class-map read)
     // design-region snapshot: E^{m+1} of the E edges in the box

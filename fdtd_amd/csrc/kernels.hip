@@ -32,54 +32,54 @@ namespace fdtd {
 // step, a launch each / one launch: 150x131x118 70 / 52, 203x149x97 with
 // magnetic classes 86 / 65, 400x130x70 82 / 67, 320x320x130 magnetic 234 /
 // 226, 512x512x64 322 / 310.
-template <class T, int CM>
+template <class T, int CM, int ST>
 __global__ void __launch_bounds__(TX * BY) E_OCC e_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x;
     int tx, ty, tz;
     if (b < ng) {
         tile_of_region<V_GEN>(a, tx, ty, tz, b);
-        e_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        e_tile<T, CM, V_GEN | ST>(a, m, tx, ty, tz);
     } else if (b < ng + nx) {
         tile_of_region<V_X>(a, tx, ty, tz, b - ng);
-        e_tile<T, CM, V_X>(a, m, tx, ty, tz);
+        e_tile<T, CM, V_X | ST>(a, m, tx, ty, tz);
     } else {
         tile_of_region<V_IN>(a, tx, ty, tz, b - ng - nx);
-        e_tile<T, CM, V_IN>(a, m, tx, ty, tz);
+        e_tile<T, CM, V_IN | ST>(a, m, tx, ty, tz);
     }
 }
-template <class T, int CM>
+template <class T, int CM, int ST>
 __global__ void __launch_bounds__(TX * BY) H_OCC h_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x;
     int tx, ty, tz;
     if (b < ng) {
         tile_of_region<V_GEN>(a, tx, ty, tz, b);
-        h_tile<T, CM, V_GEN>(a, m, tx, ty, tz);
+        h_tile<T, CM, V_GEN | ST>(a, m, tx, ty, tz);
     } else if (b < ng + nx) {
         tile_of_region<V_X>(a, tx, ty, tz, b - ng);
-        h_tile<T, CM, V_X>(a, m, tx, ty, tz);
+        h_tile<T, CM, V_X | ST>(a, m, tx, ty, tz);
     } else {
         tile_of_region<V_IN>(a, tx, ty, tz, b - ng - nx);
-        h_tile<T, CM, V_IN>(a, m, tx, ty, tz);
+        h_tile<T, CM, V_IN | ST>(a, m, tx, ty, tz);
     }
 }
 
 // ---- launchers --------------------------------------------------------------
-template <class T>
+template <class T, int ST>
 static hipError_t launch_t(bool efield, int mode, const KArgs &a, int m, hipStream_t s)
 {
     int nb, nx, nzt, ng;   // nzt = 0: the forward sweeps run without zsplit
     region_tiles(a, nb, nx, nzt, ng);
     dim3 grid(nb + nx + ng), block(TX * BY);
     if (efield) {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((e_kernel<T, CLS_UNIFORM>), grid, block, 0, s, a, m, ng, nx);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((e_kernel<T, CLS_U16>), grid, block, 0, s, a, m, ng, nx);
-        else hipLaunchKernelGGL((e_kernel<T, CLS_U32>), grid, block, 0, s, a, m, ng, nx);
+        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((e_kernel<T, CLS_UNIFORM, ST>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((e_kernel<T, CLS_U16, ST>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((e_kernel<T, CLS_U32, ST>), grid, block, 0, s, a, m, ng, nx);
     } else {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((h_kernel<T, CLS_UNIFORM>), grid, block, 0, s, a, m, ng, nx);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((h_kernel<T, CLS_U16>), grid, block, 0, s, a, m, ng, nx);
-        else hipLaunchKernelGGL((h_kernel<T, CLS_U32>), grid, block, 0, s, a, m, ng, nx);
+        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((h_kernel<T, CLS_UNIFORM, ST>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((h_kernel<T, CLS_U16, ST>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((h_kernel<T, CLS_U32, ST>), grid, block, 0, s, a, m, ng, nx);
     }
     return hipGetLastError();
 }
@@ -88,10 +88,10 @@ static hipError_t launch_t(bool efield, int mode, const KArgs &a, int m, hipStre
 hipError_t launch_half_step(bool efield, int storage, int mode, const KArgs &a, int m, hipStream_t s)
 {
     switch (storage) {
-    case 0: return launch_t<float>(efield, mode, a, m, s);
-    case 1: return launch_t<_Float16>(efield, mode, a, m, s);
-    case 2: return launch_t<bf16_t>(efield, mode, a, m, s);
-    case 3: return launch_t<bq16_t>(efield, mode, a, m, s);
+    case 0: return a.stream ? launch_t<float, V_STREAM>(efield, mode, a, m, s) : launch_t<float, 0>(efield, mode, a, m, s);
+    case 1: return a.stream ? launch_t<_Float16, V_STREAM>(efield, mode, a, m, s) : launch_t<_Float16, 0>(efield, mode, a, m, s);
+    case 2: return a.stream ? launch_t<bf16_t, V_STREAM>(efield, mode, a, m, s) : launch_t<bf16_t, 0>(efield, mode, a, m, s);
+    case 3: return a.stream ? launch_t<bq16_t, V_STREAM>(efield, mode, a, m, s) : launch_t<bq16_t, 0>(efield, mode, a, m, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -29,8 +29,21 @@ __device__ __forceinline__ std::uint32_t carry(std::uint32_t v)
     return r;
 }
 
-// Non-temporal access for the streams only the owning thread touches (the
-// swept field's own values): they are read once and written once per sweep.
+// Access to the streams only the owning thread touches (the swept field's own
+// values), which are read once and written once per sweep: non-temporal where
+// the region variant has the bit V_STREAM, else as everything.
+template <bool NT, class U>
+__device__ __forceinline__ U ldv(const U *p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, class U>
+__device__ __forceinline__ void stv(U *p, U v)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
 __device__ __forceinline__ float ldn(const float *p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void stn(float *p, float v) { __builtin_nontemporal_store(v, p); }
 __device__ __forceinline__ float ldn(const _Float16 *p) { return (float)__builtin_nontemporal_load(p); }
@@ -112,20 +125,18 @@ __device__ __forceinline__ float fldw(const T *base, std::uint32_t o, const QW<T
 {
     return ld((const T *)((const char *)base + o));
 }
-template <class T>
-__device__ __forceinline__ float fldnw(const T *base, std::uint32_t o, const QW<T> &, int)
-{
-    return ldn((const T *)((const char *)base + o));
-}
 template <>
 __device__ __forceinline__ float fldw<bq16_t>(const bq16_t *base, std::uint32_t o, const QW<bq16_t> &w, int c)
 {
     return ldexpf((float)*(const std::int16_t *)((const char *)base + o), qe(w, c));
 }
-template <>
-__device__ __forceinline__ float fldnw<bq16_t>(const bq16_t *base, std::uint32_t o, const QW<bq16_t> &w, int c)
+// The swept field's own value (NT: non-temporal)
+template <bool NT, class T>
+__device__ __forceinline__ float fldnw(const T *base, std::uint32_t o, const QW<T> &w, int c)
 {
-    return ldexpf((float)__builtin_nontemporal_load((const std::int16_t *)((const char *)base + o)), qe(w, c));
+    if constexpr (is_bq<T>::value) return ldexpf((float)ldv<NT>((const std::int16_t *)((const char *)base + o)), qe(w, c));
+    else if constexpr (NT) return ldn((const T *)((const char *)base + o));
+    else return ld((const T *)((const char *)base + o));
 }
 
 // Lane permutations within a 16-lane row (DPP, no memory access): another
@@ -162,24 +173,25 @@ __device__ __forceinline__ int bq_mantissa(float x, int e)
 // sits on lane i % 64 of its wave): the block is re-encoded with one
 // exponent from its largest magnitude, each valid cell stores upd ? v : old
 // (its current value), and the exponent's byte is returned (for stq).
-template <class T>
-__device__ __forceinline__ std::uint32_t fst(T *base, std::uint32_t o, bool upd, float v, float, bool)
+template <bool NT, class T>
+__device__ __forceinline__ std::uint32_t fst(T *base, std::uint32_t o, bool upd, float v, float old, bool valid)
 {
-    if (upd) stn((T *)((char *)base + o), v);
-    return 0;
-}
-template <>
-__device__ __forceinline__ std::uint32_t fst<bq16_t>(bq16_t *base, std::uint32_t o, bool upd, float v, float old,
-                                                     bool valid)
-{
-    const float x = !valid ? 0.f : upd ? v : old;
-    float mx = fabsf(x);
-    mx = fmaxf(mx, dpp_f<DPP_QUAD_XOR1>(mx));
-    mx = fmaxf(mx, dpp_f<DPP_QUAD_XOR2>(mx));
-    mx = fmaxf(mx, dpp_f<DPP_HALF_MIRROR>(mx));
-    const int e = bq_exponent(mx);
-    if (valid) __builtin_nontemporal_store((std::int16_t)bq_mantissa(x, e), (std::int16_t *)((char *)base + o));
-    return (std::uint32_t)(e + BQ_BIAS);
+    if constexpr (!is_bq<T>::value) {
+        if (upd) {
+            if constexpr (NT) stn((T *)((char *)base + o), v);
+            else st((T *)((char *)base + o), v);
+        }
+        return 0;
+    } else {
+        const float x = !valid ? 0.f : upd ? v : old;
+        float mx = fabsf(x);
+        mx = fmaxf(mx, dpp_f<DPP_QUAD_XOR1>(mx));
+        mx = fmaxf(mx, dpp_f<DPP_QUAD_XOR2>(mx));
+        mx = fmaxf(mx, dpp_f<DPP_HALF_MIRROR>(mx));
+        const int e = bq_exponent(mx);
+        if (valid) stv<NT>((std::int16_t *)((char *)base + o), (std::int16_t)bq_mantissa(x, e));
+        return (std::uint32_t)(e + BQ_BIAS);
+    }
 }
 
 // The three exponent bytes of a swept field at the block of byte offset o

@@ -1,5 +1,6 @@
 """GPU: a half-step's region variants in one launch, bit for bit the general
-variant over the whole grid (FDTD_INTERIOR=0): with and without interior tile
+variant over the whole grid (FDTD_INTERIOR=0), past and through the caches
+(FDTD_STREAM): with and without interior tile
 columns, a last column of one cell, odd rows, the shortest interior box, and
 grids on both sides of the 3 M-cell line of the 16-bit rule."""
 import numpy as np
@@ -20,13 +21,15 @@ def test_regions_in_one_launch(engine, monkeypatch, storage, nx, ny, nz, L):
     monkeypatch.setenv("FDTD_PERSIST", "0")
     monkeypatch.setenv("FDTD_FUSED", "0")
     got = []
-    for interior in ("0", "1"):
+    for interior, stream in (("0", "1"), ("1", "1"), ("1", "0")):
         monkeypatch.setenv("FDTD_INTERIOR", interior)
-        print(f"[regions] {storage} {nx}x{ny}x{nz} L={L} interior={interior}", flush=True)
+        monkeypatch.setenv("FDTD_STREAM", stream)
+        print(f"[regions] {storage} {nx}x{ny}x{nz} L={L} interior={interior} stream={stream}", flush=True)
         sim = engine.Simulation.from_scene(sc, storage)
         sim.run(sc.steps)
         got.append([sim.probes(), sim.dft()] + [sim.field(c) for c in range(6)])
         sim.close()
     assert min(np.count_nonzero(f) for f in got[0][2:]) > nx * ny * nz // 2   # the waves fill the grid
-    for a, b in zip(*got):
-        np.testing.assert_array_equal(a, b)
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            np.testing.assert_array_equal(a, b)
