@@ -296,12 +296,15 @@ int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_e
 // The x-edge variant takes the tiles beside the box in x, the general
 // variant the rows and z-blocks outside it.  Where no column of tiles is
 // interior (nx up to two tiles and a slab), the x-edge variant takes every
-// column of the box's rows and z-blocks, from 3 M cells on for 16-bit
-// storage: us per step, general variant alone / so: FP16 256^3 214 / 178,
-// 220x128x128 62 / 59, 150x131x118 47 / 48, block-scaled int16 261 / 223, 77 /
-// 70, 60 / 64; FP32 (64-cell tiles) 112x150x200 74 / 70, 128x128x100 38.5 /
-// 37.7.  FDTD_INTERIOR=0, or a y or z axis without interior tiles, leaves the
-// box empty (z range [0, 0)) and every tile to the general variant.
+// column of the box's rows and z-blocks -- with 128-cell tiles where they
+// leave no 64 columns idle that the general variant's 64-cell tiles would not
+// (or one in six).  us per step, general variant alone / so: FP16 220x220x200
+// 117 / 93, 250x150x60 38.6 / 36.2, 128x200x200 62 / 55; block-scaled int16
+// 220x220x200 170 / 134, 128x128x100 42.7 / 38.6; with 64 idle columns of 256
+// FP16 180x180x160 66.3 / 67.4, 160x160x150 55 / 59; FP32 112x150x200 74 / 70,
+// 100x80x70 19.9 / 18.2.  FDTD_INTERIOR=0, or a y or z axis without interior
+// tiles, leaves the box empty (z range [0, 0)) and every tile to the general
+// variant.
 // beyond: cells past the tile's high sides that must lie off the slabs too
 // (the fused step evaluates one).
 void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int beyond = 0)
@@ -324,7 +327,8 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
                 hi = t + 1;
             }
         if (hi <= lo) {
-            if (ax > 0 || sweep == 2 || (tile_cols > 64 && (double)in.nx * in.ny * in.nz < 3e6)) return;
+            const int t64 = (in.nx + 63) / 64;
+            if (ax > 0 || sweep == 2 || (tile_cols > 64 && t64 % 2 != 0 && t64 < 5)) return;
             lo = hi = 0;
         }
         box[ax] = lo;
@@ -776,7 +780,17 @@ int do_finalize(fdtd_ctx *c)
     const char *gv = std::getenv("FDTD_GEN16");
     c->pair_gen_cells = !(gv && std::strcmp(gv, "pair") == 0);
     c->pair_tiles_x = (in.nx + pair_tile_cols() - 1) / pair_tile_cols();
-    c->pair_kchunk = choose_chunks(c, c->pair_tiles_x * a.tiles_y, 8, "FDTD_PAIR_PLANES");
+    // planes in whole blocks of p off the z slabs and faces
+    auto inner = [&](int p) {
+        const int lo = std::max(in.cpml.thick[4], 1), hi = in.nz - std::max(in.cpml.thick[5], 1);
+        return std::max(0, hi / p * p - (lo + p - 1) / p * p);
+    };
+    // Block-scaled storage: 16 planes a block where as many planes stay off the
+    // general variant; us per step, 8 / 16: 512x512x256 791 / 780, 384^3 675 /
+    // 643, 256^3 212 / 205; where fewer do: 512x512x120 402 / 421, 300x200x200
+    // 147 / 149.  (FP16, where as many do: 512x512x256 657 / 668, 256^3 178 / 173.)
+    const int pp = in.storage == FDTD_STORE_BQ16 && inner(16) >= inner(8) ? 16 : 8;
+    c->pair_kchunk = choose_chunks(c, c->pair_tiles_x * a.tiles_y, pp, "FDTD_PAIR_PLANES");
     a.rec = 1;
     a.snap = nullptr;
 

@@ -769,8 +769,18 @@ __device__ __forceinline__ void h_pair_tile(const KArgs &a, const int m, const i
 // the right ones.  One launch against one for each variant, us per step (FP16):
 // 512x512x256 680 / 656, 300x200x200 163 / 140, 512x200x64 98 / 75; block-
 // scaled int16 808 / 806, 203 / 174, 123 / 95.
+// Waves per SIMD that the registers are held to: block-scaled storage in grids
+// that stream from HBM needs four (its x-edge tiles' 137 registers allow three;
+// 512x512x256 804 us a step, held to four 791, 512x512x120 414 / 402; through
+// the caches 256^3 212 / 216, 220x128x128 61.6 / 63.0).
+template <class T, int ST>
+constexpr int pair_waves()
+{
+    return is_bq<T>::value && ST ? 4 : 1;
+}
+
 template <class T, int CM, int ST, bool CELLS>
-__global__ void __launch_bounds__(TX * BY) P_OCC e_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
+__global__ void __launch_bounds__(TX * BY, (pair_waves<T, ST>())) P_OCC e_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x, n = CELLS ? 2 * ng : ng;
     int tx, ty, tz;
@@ -791,7 +801,7 @@ __global__ void __launch_bounds__(TX * BY) P_OCC e_pair_kernel(const KArgs a, co
     }
 }
 template <class T, int CM, int ST, bool CELLS>
-__global__ void __launch_bounds__(TX * BY) P_OCC h_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
+__global__ void __launch_bounds__(TX * BY, (pair_waves<T, ST>())) P_OCC h_pair_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x, n = CELLS ? 2 * ng : ng;
     int tx, ty, tz;

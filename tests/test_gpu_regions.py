@@ -2,7 +2,7 @@
 variant over the whole grid (FDTD_INTERIOR=0), past and through the caches
 (FDTD_STREAM): with and without interior tile
 columns, a last column of one cell, odd rows, the shortest interior box, and
-grids on both sides of the 3 M-cell line of the 16-bit rule."""
+16-bit grids on both sides of the rule for x-edge columns alone."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("storage,nx,ny,nz,L", [
     ("f32", 129, 61, 50, 5), ("f32", 64, 40, 37, 8), ("f32", 200, 33, 29, 3), ("f32", 193, 90, 71, 10),
     ("f16", 200, 128, 118, 7), ("f16", 129, 160, 147, 6), ("bf16", 257, 120, 100, 8), ("bf16", 130, 60, 40, 4),
-    ("bq16", 201, 130, 117, 7), ("bq16", 390, 61, 50, 5)])
+    ("bq16", 201, 130, 117, 7), ("bq16", 260, 50, 44, 6), ("bq16", 390, 61, 50, 5)])
 def test_regions_in_one_launch(engine, monkeypatch, storage, nx, ny, nz, L):
     sc = scenes.dielectric(nx=nx, ny=ny, nz=nz, steps=200, L=L, n_boxes=5, n_src=2, n_probes=6, n_freqs=2, seed=17,
                            name="regions")
