@@ -416,7 +416,7 @@ void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector
     std::vector<REvent> events;
     int max_ev = 0;
     // E events and source edges by tile
-    struct At { int i, j, k, u; Event e; };
+    struct At { int i, j, k, u; Event e; std::uint32_t cls; };
     std::vector<std::vector<At>> per(tiles);
     auto tile_of = [&](int j, int k) { return (k / tz) * gy + j / ty; };
     auto unit_of = [&](int i, int j, int k) { return ((k % tz) * ty + j % ty) * sx + i / 64; };
@@ -424,7 +424,7 @@ void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector
         if (e.kind < 0) break;   // (the H events follow)
         if (e.kind != EV_SOURCE && e.kind > EV_PROBE + 2) continue;
         const int i = e.col % nx, j = e.col / nx;
-        per[tile_of(j, e.k)].push_back(At{i, j, e.k, unit_of(i, j, e.k), e});
+        per[tile_of(j, e.k)].push_back(At{i, j, e.k, unit_of(i, j, e.k), e, bt.src_cls[&e - bt.events.data()]});
     }
     // source gathers: of the cell itself, of (i-1, j) and of (i, j-1), the
     // latter in the tile below when j is its first row
@@ -437,8 +437,7 @@ void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector
                 const int i = q == 1 ? s.i - 1 : s.i, j = q == 2 ? s.j - 1 : s.j;
                 if (i < 0 || j < 0) continue;
                 const SrcEdge &se = bt.srcs_si[s.e.id];
-                size_t cl = 0;
-                if (!bt.e_uniform && !bt.cls.empty()) cl = bt.cls[((size_t)s.k * ny + s.j) * in.px + s.i];
+                const size_t cl = bt.e_uniform ? 0 : s.cls;
                 const float *ez = bt.etab_si.data() + (cl * 3 + 2) * 4;
                 const int *L = in.cpml.thick;
                 auto slab = [](int v, int n, int lo, int hi) { return (v > 0 && v < lo) || (v >= n - hi && v < n - 1); };
@@ -913,6 +912,12 @@ int upload_tables(fdtd_ctx *c)
         a.cls = tmp;
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    b.src_cls.assign(b.events.size(), 0);
+    for (size_t q = 0; q < b.events.size() && !b.cls.empty(); ++q) {
+        const Event &e = b.events[q];
+        if (e.kind == EV_SOURCE)
+            b.src_cls[q] = b.cls[((size_t)e.k * a.ny + e.col / a.nx) * a.px + e.col % a.nx];
+    }
     std::vector<uint32_t>().swap(b.cls);   // host copy no longer needed
     return FDTD_OK;
 }

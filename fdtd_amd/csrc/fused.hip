@@ -25,8 +25,8 @@
 // What bounds it: HBM.  On 512x512x256 (CPML 16, one H class) the interior
 // tiles move 59 B per cell (50 are needed) at 5.2 TB/s, at 8, 16 or 24 waves
 // per CU alike; a bare stream of six arrays read and six written in this
-// tile order runs at 4.7 TB/s, in linear order at 5.7.  Step 1086 (two
-// sweeps) -> 947 us; 256^3 292 -> 281 us.  Tried and slower: 128 x 7 tiles
+// tile order runs at 4.7 TB/s, in linear order at 5.7.  Step 1061 (the
+// half-steps of kernels.hip, which win up to 24 M cells) -> 937 us.  Tried and slower: 128 x 7 tiles
 // (one workgroup of 16 waves per CU: 992 us), 64 x 3 (1029) and 64 x 15
 // tiles (999), z-blocks of 8 and 32 planes (977, 968), ordinary instead of
 // non-temporal stores (993), the region variants as branches of one launch

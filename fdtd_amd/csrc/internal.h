@@ -281,6 +281,7 @@ struct Built {
     std::vector<float> prof[3];     // [2n][4] per axis
     std::vector<int> e_first, h_first;
     std::vector<Event> events;
+    std::vector<std::uint32_t> src_cls;    // per event: the class of a source edge's cell (kept when cls is freed)
     std::vector<SrcEdge> srcs;
     std::vector<SrcEdge> srcs_si;   // SI coefficients (adjoint)
     int src_j0 = 1, src_j1 = 0;     // rows j whose row j or j+1 holds a source edge: [src_j0, src_j1]

@@ -29,6 +29,9 @@ def block(sc):
     i = 61 if i0 > 70 else 3 + (i0 - 5 if i0 > 9 else 0)
     sc.sources[0] = scenes.Source((i, j0 - 3, k0, i + 5 if i0 > 70 else i, j0 + 3, k0 + 3), 50.0, s0.wtype, s0.amp,
                                   s0.t0, s0.tau, s0.freq)
+    # in a lossy material (the source edges' own class is not the vacuum's)
+    sc.boxes.append(scenes.Box((i - 2, j0 - 5, k0 - 2, min(i + 8, i0 - 1), j0 + 6, k0 + 6), (2.5, 3.0, 2.0),
+                               (0.02, 0.01, 0.03)))
     sc.sources.append(scenes.z_edge(2, sc.ny // 2, sc.nz // 2, sc.dt))
     sc.probes.append((scenes.EZ, sc.probes[0][1], j0 - 1, k0))
     sc.probes.append((scenes.EX, sc.probes[0][1], j0, k0 + 1))
