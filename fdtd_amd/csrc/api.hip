@@ -389,6 +389,23 @@ void setup_fused(fdtd_ctx *c)
     c->fused = true;
 }
 
+// Give the fused step's second buffers back; the context steps with the two
+// sweeps from here on (same bits).
+void release_fused(fdtd_ctx *c)
+{
+    (void)hipStreamSynchronize(c->stream);
+    auto drop = [c](void *&p, size_t bytes) {
+        if (!p) return;
+        (void)hipFree(p);
+        c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), p));
+        c->dev_bytes -= bytes;
+        p = nullptr;
+    };
+    for (auto &f : c->fields2) drop(f, (size_t)c->field_elems * c->esz);
+    for (int p = 0; p < 12; ++p) drop(c->psi2[p], std::max<size_t>(c->psi_elems[p], 1) * c->esz);
+    c->fused = false;
+}
+
 // Reverse steps in one launch: on the tiles of the forward ones (ty x tz rows
 // of sx segments, gy of them along y), whose exchange rows are taken from the
 // forward units.  Rule: wherever the forward steps run in one launch and a
@@ -1307,6 +1324,10 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
         HIPCHK(c, hipMemGetInfo(&freeb, &totb));
         const size_t need = nhist * hist_bytes + (size_t)(nseg - 1) * ck_bytes + adj_bytes +
                             (size_t)np * n * 4 + 3 * nb * 8;
+        if ((double)need > 0.9 * (double)freeb && c->fused) {   // (memory before the one-pass step)
+            release_fused(c);
+            HIPCHK(c, hipMemGetInfo(&freeb, &totb));
+        }
         if ((double)need > 0.9 * (double)freeb)
             return fail(c, FDTD_E_NOMEM, "adjoint needs %.2f GB of device memory, %.2f GB free; use a larger "
                         "checkpoint interval", need / 1e9, freeb / 1e9);

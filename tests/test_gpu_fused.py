@@ -85,3 +85,26 @@ def test_adjoint_with_the_fused_forward(engine, monkeypatch, every):
         sim.close()
     assert got[0][0] == got[1][0] and got[0][0] > 0
     np.testing.assert_array_equal(got[0][1], got[1][1])
+
+
+def test_second_buffers_are_given_back(engine, monkeypatch):
+    """An adjoint that does not fit takes the memory of the one-pass step's
+    second buffers before it is refused; the context steps on with the sweeps."""
+    sc = scenes.adjoint(nx=80, ny=80, nz=72, steps=400000, L=5, design=(40, 40, 40), n_probes=1, probe_freqs=(5e9,),
+                        seed=9)
+    got = []
+    for fused in ("0", "1"):
+        monkeypatch.setenv("FDTD_FUSED", fused)
+        sim = engine.Simulation.from_scene(sc, "f32")
+        print(f"[fused] adjoint refused, fused={fused}", flush=True)
+        sim.run(20)
+        before = sim.info()["device_bytes"]
+        with pytest.raises(engine.FdtdError) as ei:
+            sim.adjoint_gradient([(0, 0, 1.0)], sc.steps, 0)   # a 331 GB history
+        assert ei.value.code == -4 and "use a larger" in str(ei.value)
+        assert (sim.info()["device_bytes"] < before) == (fused == "1")
+        sim.run(20)
+        got.append([sim.field(c) for c in range(6)])
+        sim.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
