@@ -1408,13 +1408,15 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     // disables): its tile columns and the others, and the second dJ/dE,
     // dJ/dH buffers it writes (the pair is swapped after every step).  Not
     // with the no-allocation scratch, nor when the pair would take more than
-    // half the free memory.
+    // half the free memory, nor where all steps of a segment run in one launch
+    // (in place: a swap would leave the next segment the zeros of the second
+    // buffers).
     bool pp = false;
     {
         const char *fv = std::getenv("FDTD_ADJ_FUSE");
         const bool want = !(fv && std::strcmp(fv, "0") == 0);
         std::vector<int> quiet, noisy;
-        if (want && !arena && huni && !adj_stores_quantities(nx) && aa.ib[0] >= 0)
+        if (want && !arena && !radj && huni && !adj_stores_quantities(nx) && aa.ib[0] >= 0)
             adj_fuse_tiles(aa, c->built.e_first, c->built.h_first, b.sb, quiet, noisy);
         const size_t pair_bytes = 6 * (size_t)c->field_elems * 4 + (quiet.size() + noisy.size() + 2) * 4;
         if (!quiet.empty()) HIPCHK(c, hipMemGetInfo(&freeb, &totb));
