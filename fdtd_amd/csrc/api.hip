@@ -65,6 +65,7 @@ struct fdtd_ctx {
     KArgs ka{};
     int e_mode = 0, h_mode = 0;
     int steps_done = 0;
+    bool broken = false;            // a launch gave up a wait: no valid state until a reset or a restore
     bool has_port = false;          // fdtd_set_port: its samples are probes port_base ..
     int port_base = 0;
     PortPlan port;
@@ -258,6 +259,7 @@ int zero_state(fdtd_ctx *c)
     if (np && nf) HIPCHK(c, hipMemsetAsync(c->ka.dft, 0, np * nf * sizeof(double2), c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->steps_done = 0;
+    c->broken = false;
     return FDTD_OK;
 }
 
@@ -558,7 +560,6 @@ void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector
     r.units = U;
     r.cls16 = c->pa.cls16;
     r.euni = bt.e_uniform ? 1 : 0;
-    r.max_polls = c->pa.max_polls;
     r.failed = c->pa.failed;
     r.ll = c->pa.ll;
     r.tiles = (const PTile *)dt;
@@ -566,6 +567,14 @@ void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector
     r.events = (const REvent *)de;
     c->rlds = lds;
     c->radj = true;
+}
+
+// Reads of a neighbour's row before a wait is given up (some seconds);
+// FDTD_PERSIST_POLLS, looked up at each launch, overrides it.
+int poll_limit()
+{
+    const char *mp = std::getenv("FDTD_PERSIST_POLLS");
+    return mp ? std::atoi(mp) : 1 << 22;
 }
 
 // Tiles, exchange rows and event lists of the steps in one launch; a context
@@ -723,8 +732,7 @@ void setup_persist(fdtd_ctx *c)
     p.units = U;
     p.cls16 = c->built.mode == CLS_U16 ? 1 : 0;
     p.epoch = 1;
-    const char *mp = std::getenv("FDTD_PERSIST_POLLS");
-    p.max_polls = mp ? std::atoi(mp) : 1 << 22;   // some seconds
+    p.max_polls = poll_limit();
     p.failed = (int *)fd;
     p.ll = (std::uint64_t *)ll;
     p.tiles = (const PTile *)dt;
@@ -1044,20 +1052,32 @@ hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
     bind_sets(c, a);
     p.m0 = m0;
     p.n = n;
+    p.max_polls = poll_limit();
     if ((e = launch_persist(c->in.storage, a, p, c->ptiles, c->plds, c->stream)) != hipSuccess) return e;
     p.epoch += (std::uint32_t)n + 1u;
     return a.rec ? launch_dft(a, (int)c->in.probes.size(), m0, n, c->stream) : hipSuccess;
 }
 
-// After a synchronisation: whether a launch of advance gave up a wait.
+// A context whose last launch gave up a wait holds no state to run on, read
+// or save.
+int check_state(fdtd_ctx *c)
+{
+    return c->broken ? fail(c, FDTD_E_STATE, "the state is not valid: a launch gave up a wait (fdtd_reset or "
+                            "fdtd_checkpoint_restore starts over)") : FDTD_OK;
+}
+
+// After a synchronisation: whether a launch of advance gave up a wait.  The
+// flag and the exchange rows are cleared in the order of the context's stream
+// (it does not wait for the null stream's work).
 int check_advance(fdtd_ctx *c)
 {
     if (!c->persist) return FDTD_OK;
     int failed = 0;
     HIPCHK(c, hipMemcpy(&failed, c->pa.failed, sizeof failed, hipMemcpyDeviceToHost));
     if (!failed) return FDTD_OK;
-    HIPCHK(c, hipMemset(c->pa.failed, 0, sizeof failed));
-    HIPCHK(c, hipMemset(c->pa.ll, 0, c->pll));
+    c->broken = true;
+    HIPCHK(c, hipMemsetAsync(c->pa.failed, 0, sizeof failed, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->pa.ll, 0, c->pll, c->stream));
     c->pa.epoch = 1;
     return fail(c, FDTD_E_DEVICE, "a workgroup waited too long for a neighbour's rows; the state is not valid "
                 "(fdtd_reset starts over)");
@@ -1101,6 +1121,7 @@ struct EventSet {
 int run_steps(fdtd_ctx *c, int nsteps, bool profile)
 {
     if (!c->finalized) return fail(c, FDTD_E_STATE, "fdtd_finalize has not been called");
+    if (int rc = check_state(c)) return rc;
     if (nsteps < 0) return fail(c, FDTD_E_INVALID, "nsteps < 0");
     if (c->steps_done + nsteps > c->in.steps_cap)
         return fail(c, FDTD_E_RANGE, "run past the finalized horizon (%d + %d > %d)", c->steps_done, nsteps,
@@ -1566,6 +1587,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
             HIPCHK(c, new_epochs(c, s1 - s0));
             r.m1 = s1 - 1;
             r.n = s1 - s0;
+            r.max_polls = poll_limit();
             r.epoch = c->pa.epoch;
             HIPCHK(c, launch_adj_persist(aa, b, r, c->ptiles, c->rlds, rs));
             c->pa.epoch += (std::uint32_t)r.n + 1u;
@@ -1960,6 +1982,7 @@ int fdtd_get_probes(fdtd_ctx *c, float *out, size_t n)
 {
     if (!c || (!out && n)) return FDTD_E_INVALID;
     if (!c->finalized) return fail(c, FDTD_E_STATE, "not finalized");
+    if (int rc = check_state(c)) return rc;
     const size_t np = c->in.probes.size(), ns = (size_t)c->steps_done;
     if (n < np * ns) return fail(c, FDTD_E_INVALID, "output holds %zu values, need %zu", n, np * ns);
     if (np && ns)
@@ -1991,6 +2014,7 @@ static int port_read(fdtd_ctx *c, std::vector<float> &v, std::vector<float> &cur
 {
     if (!c->finalized) return fail(c, FDTD_E_STATE, "not finalized");
     if (!c->has_port) return fail(c, FDTD_E_STATE, "no port was set");
+    if (int rc = check_state(c)) return rc;
     const size_t np = c->port.samples.size(), ns = (size_t)c->steps_done;
     v.assign(ns, 0.f);
     cur.assign(ns, 0.f);
@@ -2038,6 +2062,7 @@ int fdtd_get_dft(fdtd_ctx *c, double *out, size_t n)
 {
     if (!c || (!out && n)) return FDTD_E_INVALID;
     if (!c->finalized) return fail(c, FDTD_E_STATE, "not finalized");
+    if (int rc = check_state(c)) return rc;
     const size_t cnt = c->in.probes.size() * c->in.freqs.size() * 2;
     if (n < cnt) return fail(c, FDTD_E_INVALID, "output holds %zu values, need %zu", n, cnt);
     if (cnt) HIPCHK(c, hipMemcpy(out, c->ka.dft, cnt * sizeof(double), hipMemcpyDeviceToHost));
@@ -2048,6 +2073,7 @@ int fdtd_get_field(fdtd_ctx *c, int comp, float *out, size_t n)
 {
     if (!c || !out) return FDTD_E_INVALID;
     if (!c->finalized) return fail(c, FDTD_E_STATE, "not finalized");
+    if (int rc = check_state(c)) return rc;
     if (comp < 0 || comp > 5) return fail(c, FDTD_E_INVALID, "invalid component");
     const int nx = c->in.nx, ny = c->in.ny, nz = c->in.nz, px = c->in.px;
     const size_t cells = (size_t)nx * ny * nz;
@@ -2105,6 +2131,7 @@ int fdtd_checkpoint_save(fdtd_ctx *c, void *buf, size_t bytes)
     size_t need = 0;
     int rc = fdtd_checkpoint_size(c, &need);
     if (rc) return fail(c, rc, "not finalized");
+    if ((rc = check_state(c))) return rc;
     if (bytes < need) return fail(c, FDTD_E_INVALID, "checkpoint buffer holds %zu bytes, need %zu", bytes, need);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     unsigned char *p = (unsigned char *)buf + sizeof(CkHeader);
@@ -2168,6 +2195,7 @@ int fdtd_checkpoint_restore(fdtd_ctx *c, const void *buf, size_t bytes)
     if ((rc = put(c->ka.probe_hist, c->in.probes.size() * (size_t)c->in.steps_cap * sizeof(float)))) return rc;
     if ((rc = put(c->ka.dft, c->in.probes.size() * c->in.freqs.size() * sizeof(double2)))) return rc;
     c->steps_done = h.step;
+    c->broken = false;
     return FDTD_OK;
 }
 
