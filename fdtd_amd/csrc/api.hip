@@ -97,6 +97,7 @@ struct fdtd_ctx {
     // many steps in one launch (persist.hip): its arguments, tiles, LDS bytes
     // and the exchange rows' bytes
     bool persist = false;
+    bool unchecked = false;         // a launch that waits was made since its flag was read
     PArgs pa{};
     int ptiles = 0;
     size_t plds = 0, pll = 0;
@@ -226,7 +227,7 @@ void free_device(fdtd_ctx *c)
     for (auto &q : c->qarr) q = nullptr;
     for (auto &f : c->fields2) f = nullptr;
     for (auto &p : c->psi2) p = nullptr;
-    c->fused = c->persist = c->radj = false;
+    c->fused = c->persist = c->radj = c->unchecked = false;
 }
 
 // The buffers holding the current state.
@@ -585,9 +586,8 @@ int poll_limit()
 // P_MAX_EVENTS source edges and probes.  Every such grid measured is faster in
 // one launch, us per step, sweeps / one launch of 300 steps: 64^3 13.5 / 3.9,
 // 300x60x40 34.7 / 11.3, 110x150x53 27.1 / 15.2, 128x128x64 27.8 / 14.6 (FP16
-// 23.0 / 16.7), 128x128x80 32.8 / 17.1, 12x9x8 10.0 / 3.2; and from few steps:
-// 8 steps of 64^3 13.0 / 7.0, of 128x128x64 28.0 / 19.0 (the launch, loading
-// and storing the tiles take about 25 us).  FDTD_PERSIST=0 turns it off.
+// 23.0 / 16.7), 128x128x80 32.8 / 17.1, 12x9x8 10.0 / 3.2; and from 6 to 10 steps
+// on (persist_min_steps).  FDTD_PERSIST=0 turns it off.
 void setup_persist(fdtd_ctx *c)
 {
     const SceneIn &in = c->in;
@@ -1027,9 +1027,18 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
 
 constexpr size_t STAGE = 1 << 20;   // floats of a piece of fdtd_get_field
 
-// Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
-// and the call enough steps to pay for it.
-constexpr int P_MIN_STEPS = 4;
+// The fewest steps that pay for one launch -- the launch itself, loading and
+// storing the tiles, reading its flag -- by the units a wave holds.  us per
+// fdtd_run, launched / in one launch, around the line: 64^3 (one unit) 5 steps 103
+// / 108, 6 steps 115 / 112; 64x120x60 (two) 122 / 123, 138 / 129; 300x60x40 (three)
+// 6 steps 153 / 160, 7 steps 171 / 170, FP16 169 / 174, 190 / 187; 128x128x64 (four)
+// 8 steps 205 / 211, 9 steps 225 / 225; 100x96x90 (five) 9 steps 215 / 215, 10
+// steps 234 / 228.
+int persist_min_steps(const fdtd_ctx *c)
+{
+    static const int least[5] = {6, 6, 7, 9, 10};
+    return least[std::min(4, (c->pa.units - 1) / (persist_max_units() / 5))];
+}
 
 // Before a launch of n steps: start over when the step numbers run out.
 hipError_t new_epochs(fdtd_ctx *c, int n)
@@ -1039,10 +1048,12 @@ hipError_t new_epochs(fdtd_ctx *c, int n)
     return hipMemsetAsync(c->pa.ll, 0, c->pll, c->stream);
 }
 
+// Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
+// and the call enough steps.
 hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
 {
     hipError_t e = hipSuccess;
-    if (!c->persist || base.lc[3] > 0 || n < P_MIN_STEPS) {
+    if (!c->persist || base.lc[3] > 0 || n < persist_min_steps(c)) {
         for (int m = m0; m < m0 + n && e == hipSuccess; ++m) e = do_step(c, base, m);
         return e;
     }
@@ -1054,6 +1065,7 @@ hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
     p.n = n;
     p.max_polls = poll_limit();
     if ((e = launch_persist(c->in.storage, a, p, c->ptiles, c->plds, c->stream)) != hipSuccess) return e;
+    c->unchecked = true;
     p.epoch += (std::uint32_t)n + 1u;
     return a.rec ? launch_dft(a, (int)c->in.probes.size(), m0, n, c->stream) : hipSuccess;
 }
@@ -1071,9 +1083,10 @@ int check_state(fdtd_ctx *c)
 // (it does not wait for the null stream's work).
 int check_advance(fdtd_ctx *c)
 {
-    if (!c->persist) return FDTD_OK;
+    if (!c->unchecked) return FDTD_OK;
     int failed = 0;
     HIPCHK(c, hipMemcpy(&failed, c->pa.failed, sizeof failed, hipMemcpyDeviceToHost));
+    c->unchecked = false;
     if (!failed) return FDTD_OK;
     c->broken = true;
     HIPCHK(c, hipMemsetAsync(c->pa.failed, 0, sizeof failed, c->stream));
@@ -1590,6 +1603,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
             r.max_polls = poll_limit();
             r.epoch = c->pa.epoch;
             HIPCHK(c, launch_adj_persist(aa, b, r, c->ptiles, c->rlds, rs));
+            c->unchecked = true;
             c->pa.epoch += (std::uint32_t)r.n + 1u;
         }
         for (int m = s1 - 1; !radj && m >= s0; --m) {
