@@ -1034,10 +1034,11 @@ constexpr size_t STAGE = 1 << 20;   // floats of a piece of fdtd_get_field
 // 6 steps 153 / 160, 7 steps 171 / 170, FP16 169 / 174, 190 / 187; 128x128x64 (four)
 // 8 steps 205 / 211, 9 steps 225 / 225; 100x96x90 (five) 9 steps 215 / 215, 10
 // steps 234 / 228.
+int units_per_wave(const fdtd_ctx *c) { return (5 * c->pa.units - 1) / persist_max_units() + 1; }
 int persist_min_steps(const fdtd_ctx *c)
 {
     static const int least[5] = {6, 6, 7, 9, 10};
-    return least[std::min(4, (c->pa.units - 1) / (persist_max_units() / 5))];
+    return least[units_per_wave(c) - 1];
 }
 
 // Before a launch of n steps: start over when the step numbers run out.
@@ -1049,11 +1050,11 @@ hipError_t new_epochs(fdtd_ctx *c, int n)
 }
 
 // Steps m0 .. m0 + n - 1, in one launch where the context has the tiles for it
-// and the call enough steps.
-hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n)
+// and the call `least` steps.
+hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n, int least)
 {
     hipError_t e = hipSuccess;
-    if (!c->persist || base.lc[3] > 0 || n < persist_min_steps(c)) {
+    if (!c->persist || base.lc[3] > 0 || n < least) {
         for (int m = m0; m < m0 + n && e == hipSuccess; ++m) e = do_step(c, base, m);
         return e;
     }
@@ -1146,7 +1147,7 @@ int run_steps(fdtd_ctx *c, int nsteps, bool profile)
     hipEvent_t *evs = all.v.data() + 2;
     const int m0 = c->steps_done;
     HIPCHK(c, hipEventRecord(t0, c->stream));
-    if (!profile) HIPCHK(c, advance(c, c->ka, m0, nsteps));
+    if (!profile) HIPCHK(c, advance(c, c->ka, m0, nsteps, persist_min_steps(c)));
     for (int s = 0; profile && s < nsteps; ++s)
         HIPCHK(c, do_step(c, c->ka, m0 + s, evs[4 * s + 0], evs[4 * s + 1], evs[4 * s + 2], evs[4 * s + 3]));
     HIPCHK(c, hipEventRecord(t1, c->stream));
@@ -1314,10 +1315,6 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     const int n = n_steps;
     const int bx = dnx + 1, by = dny + 1, bz = dnz + 1;
     const i64 nb = (i64)bx * by * bz;
-    // all reverse steps of a segment in one launch (a switch of the launched
-    // sweeps asks for those)
-    const bool radj = c->radj && !std::getenv("FDTD_ADJ_GATHER") && !std::getenv("FDTD_ADJ_CHUNKS") &&
-                      !std::getenv("FDTD_INTERIOR");
     // adjoint fields (6) and, on narrow grids, every cell's transposed
     // quantities (12 arrays), guard planes included
     const int nq = adj_stores_quantities(nx) ? 12 : 0;
@@ -1337,10 +1334,29 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     }
     int Kseg = K > 0 ? std::min(K, n) : n;
     const int nseg = (n + Kseg - 1) / Kseg;
+    // Small grids: the recompute of a segment in one launch where its steps pay
+    // for one (no flag is read after it, so from 4 steps on up to two units a
+    // wave), before the reverse steps on the one stream: it holds every CU's LDS,
+    // and beside it they slow down by more than it hides.  Shorter segments sweep
+    // the light cone.  ms of a gradient of 128 steps, design 6x6x6 (64^3: 8x8x8),
+    // in one launch / light cone, by segment length: 64^3 (one unit) 4: 8.7 / 9.1,
+    // 6: 6.9 / 7.3, 16: 4.1 / 5.4; 300x60x40 (three) 6: 10.9 / 10.3, 8: 9.3 / 9.3, 16:
+    // 7.7 / 8.1; 128x128x64 (four) 8: 11.2 / 10.9, 16: 9.1 / 9.5, 64: 7.9 / 9.1; 100x96x90
+    // (five) 8: 11.7 / 11.7, 16: 9.5 / 10.2.
+    const int upw = c->persist ? units_per_wave(c) : 0;
+    const int least = !c->persist ? 0 : upw <= 2 ? 4 : persist_min_steps(c);
+    const bool whole = c->persist && Kseg >= least;
+    // All reverse steps of a segment in one launch (a switch of the launched sweeps
+    // asks for those), but not of segments of one step, or two up to two units a
+    // wave: launched beside the recompute / in one launch after it, ms as above,
+    // of one step: 64^3 20.8 / 22.4, 100x96x90 27.3 / 30.9, 128x128x64 27.9 / 28.9; of
+    // two: 64^3 12.6 / 13.0, 28x24x22 12.0 / 12.4, 128x128x64 19.4 / 18.8.
+    const bool radj = c->radj && Kseg > (upw <= 2 ? 2 : 1) && !std::getenv("FDTD_ADJ_GATHER") && !std::getenv("FDTD_ADJ_CHUNKS") &&
+                      !std::getenv("FDTD_INTERIOR");
     const size_t hist_bytes = (size_t)(Kseg + 1) * 3 * nb * sizeof(float);
     const size_t ck_bytes = state_bytes(c);
-    // segmented runs double-buffer the history: segment s-1 is recomputed on
-    // a second stream while the reverse sweep of segment s runs
+    // segmented runs double-buffer the history: with launched reverse sweeps,
+    // segment s-1 is recomputed beside the reverse sweep of segment s
     const int nhist = nseg > 1 ? 2 : 1;
     if (arena) {
         if (nseg > 1)
@@ -1487,10 +1503,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     EventSet sync;
     hipStream_t rs = c->stream;
     if (nseg > 1) {
-        // (a recompute in one launch holds every CU's LDS: beside it the
-        // reverse sweeps slow down by more than it hides, so it runs before
-        // them on the one stream)
-        if (!c->persist) {
+        if (!whole && !radj) {
             HIPCHK(c, hipStreamCreateWithFlags(&rsg.s, hipStreamNonBlocking));
             rs = rsg.s;
         }
@@ -1506,7 +1519,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     for (int m = 0; m < n; m += Kseg) {
         if (nseg > 1 && m > 0)
             if ((rc = copy_state(c, pool + (size_t)(m / Kseg - 1) * ck_bytes, true))) return rc;
-        HIPCHK(c, advance(c, fa, m, std::min(Kseg, n - m)));
+        HIPCHK(c, advance(c, fa, m, std::min(Kseg, n - m), least));
     }
     HIPCHK(c, hipEventRecord(t1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1544,8 +1557,7 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     // first box for every step.  Cells outside it keep stale values, and every
     // segment restarts from a full checkpoint.
     const char *lce = std::getenv("FDTD_LIGHTCONE");
-    // (a grid that steps in one launch recomputes whole: cheaper than the box's sweeps)
-    const bool lc_on = nseg > 1 && !c->persist && !(lce && std::strcmp(lce, "0") == 0);
+    const bool lc_on = nseg > 1 && !whole && !(lce && std::strcmp(lce, "0") == 0);
     const bool lc_fixed = lce && std::strcmp(lce, "fixed") == 0;
     // the box dilated by R, or all zero (the whole grid)
     auto cone = [&](int R, int lc[6]) {
@@ -1583,8 +1595,8 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
             // snapshots of steps m .. s1-1, so the design box dilated by
             // s1 - m + 2 (Kseg + 2 at most) suffices
             if (!lc_fixed) cone(s1 - m + 2, ra.lc);
-            if (c->persist && ra.lc[3] == 0) runs = s1 - m;   // whole-grid steps, one launch
-            HIPCHK(c, advance(c, ra, m, runs));
+            if (whole) runs = s1 - m;
+            HIPCHK(c, advance(c, ra, m, runs, least));
         }
         HIPCHK(c, hipEventRecord(sync.v[q], c->stream));   // buffer q ready
         return FDTD_OK;
