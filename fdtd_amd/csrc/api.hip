@@ -74,6 +74,7 @@ struct fdtd_ctx {
     i64 field_elems = 0;            // per field allocation, guard planes included
     std::vector<void *> allocs;     // every device allocation
     long n_allocs = 0;              // device allocations attempted (failure injection)
+    long n_coops = 0;               // cooperative launches attempted (likewise)
     // Field and psi allocation bases (the sweeps update them in place).
     void *fields[6] = {};
     void *psi[12] = {};
@@ -578,6 +579,28 @@ int poll_limit()
     return mp ? std::atoi(mp) : 1 << 22;
 }
 
+// Failure injection: FDTD_FAIL_COOP=n makes the context's n-th cooperative launch
+// (the first is the trial of setup_persist) fail as refused.
+bool coop_refused(fdtd_ctx *c)
+{
+    ++c->n_coops;
+    const char *fc = std::getenv("FDTD_FAIL_COOP");
+    return fc && std::atol(fc) == c->n_coops;
+}
+
+// Many steps in one launch; one that is refused (nothing has run then) leaves
+// the context to the sweeps from here on, as at set-up.
+hipError_t launch_steps(fdtd_ctx *c, const KArgs &a)
+{
+    const hipError_t e = coop_refused(c) ? hipErrorCooperativeLaunchTooLarge
+                                         : launch_persist(c->in.storage, a, c->pa, c->ptiles, c->plds, c->stream);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        c->persist = c->radj = false;
+    }
+    return e;
+}
+
 // Tiles, exchange rows and event lists of the steps in one launch; a context
 // they do not fit, or without the memory, steps with the sweeps.
 //
@@ -747,9 +770,7 @@ void setup_persist(fdtd_ctx *c)
     KArgs ka = c->ka;
     bind_sets(c, ka);
     ka.snap = nullptr;
-    if (launch_persist(in.storage, ka, p, tiles, lds, c->stream) != hipSuccess ||
-        hipStreamSynchronize(c->stream) != hipSuccess)
-        return drop();
+    if (launch_steps(c, ka) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) return drop();
     p.epoch += 1;
     c->persist = true;
     if (!in.design_eps.empty()) setup_radj(c, pt, units, gy, tz);
@@ -1054,21 +1075,22 @@ hipError_t new_epochs(fdtd_ctx *c, int n)
 hipError_t advance(fdtd_ctx *c, const KArgs &base, int m0, int n, int least)
 {
     hipError_t e = hipSuccess;
-    if (!c->persist || base.lc[3] > 0 || n < least) {
-        for (int m = m0; m < m0 + n && e == hipSuccess; ++m) e = do_step(c, base, m);
-        return e;
+    if (c->persist && base.lc[3] == 0 && n >= least) {
+        PArgs &p = c->pa;
+        if ((e = new_epochs(c, n)) != hipSuccess) return e;
+        KArgs a = base;
+        bind_sets(c, a);
+        p.m0 = m0;
+        p.n = n;
+        p.max_polls = poll_limit();
+        if (launch_steps(c, a) == hipSuccess) {
+            c->unchecked = true;
+            p.epoch += (std::uint32_t)n + 1u;
+            return a.rec ? launch_dft(a, (int)c->in.probes.size(), m0, n, c->stream) : hipSuccess;
+        }
     }
-    PArgs &p = c->pa;
-    if ((e = new_epochs(c, n)) != hipSuccess) return e;
-    KArgs a = base;
-    bind_sets(c, a);
-    p.m0 = m0;
-    p.n = n;
-    p.max_polls = poll_limit();
-    if ((e = launch_persist(c->in.storage, a, p, c->ptiles, c->plds, c->stream)) != hipSuccess) return e;
-    c->unchecked = true;
-    p.epoch += (std::uint32_t)n + 1u;
-    return a.rec ? launch_dft(a, (int)c->in.probes.size(), m0, n, c->stream) : hipSuccess;
+    for (int m = m0; m < m0 + n && e == hipSuccess; ++m) e = do_step(c, base, m);
+    return e;
 }
 
 // A context whose last launch gave up a wait holds no state to run on, read
@@ -1269,11 +1291,14 @@ struct DevBuf {
 
 }  // namespace
 
+// Reverse steps in one launch were refused: the call starts over without them.
+constexpr int ADJ_AGAIN = 1;
+
 // arena: nullptr allocates the call's buffers with hipMalloc; otherwise they
 // are carved from arena (the static scratch, arena_cap bytes), which allows
 // one segment only (no checkpoint pool, no second stream).
-int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, double *J_out, double *grad_out,
-                size_t n_grad, unsigned char *arena = nullptr, size_t arena_cap = 0)
+static int adjoint_call(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, double *J_out, double *grad_out,
+                        size_t n_grad, unsigned char *arena, size_t arena_cap)
 {
     if (!c->finalized) return fail(c, FDTD_E_STATE, "fdtd_finalize has not been called");
     const SceneIn &in = c->in;
@@ -1614,7 +1639,11 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
             r.n = s1 - s0;
             r.max_polls = poll_limit();
             r.epoch = c->pa.epoch;
-            HIPCHK(c, launch_adj_persist(aa, b, r, c->ptiles, c->rlds, rs));
+            if (coop_refused(c) || launch_adj_persist(aa, b, r, c->ptiles, c->rlds, rs) != hipSuccess) {
+                (void)hipGetLastError();
+                c->persist = c->radj = false;
+                return ADJ_AGAIN;
+            }
             c->unchecked = true;
             c->pa.epoch += (std::uint32_t)r.n + 1u;
         }
@@ -1669,6 +1698,13 @@ int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, doub
     // when there was a single segment; otherwise rewind it
     if (nseg > 1) return zero_state(c);
     return FDTD_OK;
+}
+
+int run_adjoint(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int K, double *J_out, double *grad_out,
+                size_t n_grad, unsigned char *arena = nullptr, size_t arena_cap = 0)
+{
+    const int rc = adjoint_call(c, obj, n_steps, K, J_out, grad_out, n_grad, arena, arena_cap);
+    return rc == ADJ_AGAIN ? adjoint_call(c, obj, n_steps, K, J_out, grad_out, n_grad, arena, arena_cap) : rc;
 }
 
 // ============================================================================
