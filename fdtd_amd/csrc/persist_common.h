@@ -13,6 +13,7 @@ typedef std::uint32_t u32;
 typedef std::uint64_t u64;
 
 constexpr int PW = 16;   // waves per workgroup
+constexpr int COOP_LDS_MAX = 160 * 1024;   // bytes of a workgroup
 
 __device__ __forceinline__ void ll_put(u64 *p, float v, u32 tag)
 {
@@ -76,13 +77,15 @@ struct PDesc {
 };
 
 // Whether `tiles` workgroups of PW waves with `lds` bytes each can be
-// resident at once (and the kernel is set up to use them).
+// resident at once (and the kernel is set up to use them: its limit of dynamic
+// LDS is one of the process, so it is set to the most that any context asks for).
 inline bool coop_fits(const void *fn, int tiles, size_t lds, int device)
 {
     int coop = 0, cus = 0, per = 0;
-    bool ok = fn && hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess && coop &&
+    bool ok = fn && lds <= (size_t)COOP_LDS_MAX &&
+              hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess && coop &&
               hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-              hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
+              hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, COOP_LDS_MAX) == hipSuccess &&
               hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, 64 * PW, lds) == hipSuccess;
     if (!ok) (void)hipGetLastError();
     return ok && per >= 1 && tiles <= cus * per;
