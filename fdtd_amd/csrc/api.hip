@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <new>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -341,6 +342,14 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
     for (int q = 0; q < 6; ++q) ib[q] = box[q];
 }
 
+// Whether one of the switches is set.
+bool any_set(std::initializer_list<const char *> names)
+{
+    for (const char *n : names)
+        if (std::getenv(n)) return true;
+    return false;
+}
+
 // The fused step's tiling and its second buffers; without the memory for
 // them the context steps with the two sweeps.
 //
@@ -354,7 +363,8 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
 // / 409, 512x300x150 380 / 363, 260x260x300 376 / 398, 320x320x160 254 / 271,
 // 256^3 262 / 277.  Magnetic 512x512x256 1094 / 1081, 640x400x256 1055 / 993;
 // below 512x512x200 900 / 922, 512x512x128 573 / 634, 256^3 280 / 328.
-// FDTD_FUSED=0 / 1 overrides it.  Blocks of 16 planes, halved until a launch
+// FDTD_FUSED=0 / 1 overrides it; a switch that only the sweeps have asks for
+// those.  Blocks of 16 planes, halved until a launch
 // has 4096 workgroups (256^3: 8 planes 281 us, 16 planes 296).
 void setup_fused(fdtd_ctx *c)
 {
@@ -363,6 +373,7 @@ void setup_fused(fdtd_ctx *c)
     const char *fv = std::getenv("FDTD_FUSED");
     const bool force = fv && std::strcmp(fv, "1") == 0;
     if (in.storage != FDTD_STORE_F32 || (fv && std::strcmp(fv, "0") == 0)) return;
+    if (!force && any_set({"FDTD_STREAM", "FDTD_E_PLANES", "FDTD_H_PLANES"})) return;
     const int by = fused_rows(), tx = (in.nx + tile_cols() - 1) / tile_cols(), ty = (in.ny + by - 1) / by;
     c->kchunk_f = choose_chunks(c, tx * ty, 16, "FDTD_F_PLANES", 4096);
     sweep_split(c, 2, tile_cols(), by, c->kchunk_f, 1);
@@ -610,13 +621,16 @@ hipError_t launch_steps(fdtd_ctx *c, const KArgs &a)
 // one launch, us per step, sweeps / one launch of 300 steps: 64^3 13.5 / 3.9,
 // 300x60x40 34.7 / 11.3, 110x150x53 27.1 / 15.2, 128x128x64 27.8 / 14.6 (FP16
 // 23.0 / 16.7), 128x128x80 32.8 / 17.1, 12x9x8 10.0 / 3.2; and from 6 to 10 steps
-// on (persist_min_steps).  FDTD_PERSIST=0 turns it off.
+// on (persist_min_steps).  FDTD_PERSIST=0 turns it off, and so does a switch of
+// the launched sweeps, which asks for those.
 void setup_persist(fdtd_ctx *c)
 {
     const SceneIn &in = c->in;
     c->persist = c->radj = false;
     const char *ev = std::getenv("FDTD_PERSIST");
-    if (in.storage == FDTD_STORE_BQ16 || c->h_mode != CLS_UNIFORM || c->fused || (ev && std::strcmp(ev, "0") == 0))
+    if (in.storage == FDTD_STORE_BQ16 || c->h_mode != CLS_UNIFORM || c->fused || (ev && std::strcmp(ev, "0") == 0) ||
+        any_set({"FDTD_PAIR", "FDTD_GEN16", "FDTD_CHUNKS", "FDTD_INTERIOR", "FDTD_STREAM", "FDTD_MIN_WG",
+                 "FDTD_E_PLANES", "FDTD_H_PLANES", "FDTD_PAIR_PLANES"}))
         return;
     // the tiling: at most one tile per CU and 160 KB of LDS each, the fewest
     // units (64-cell row segments) per tile, then the fewest rows exchanged
@@ -1376,8 +1390,8 @@ static int adjoint_call(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int
     // wave: launched beside the recompute / in one launch after it, ms as above,
     // of one step: 64^3 20.8 / 22.4, 100x96x90 27.3 / 30.9, 128x128x64 27.9 / 28.9; of
     // two: 64^3 12.6 / 13.0, 28x24x22 12.0 / 12.4, 128x128x64 19.4 / 18.8.
-    const bool radj = c->radj && Kseg > (upw <= 2 ? 2 : 1) && !std::getenv("FDTD_ADJ_GATHER") && !std::getenv("FDTD_ADJ_CHUNKS") &&
-                      !std::getenv("FDTD_INTERIOR");
+    const bool radj = c->radj && Kseg > (upw <= 2 ? 2 : 1) &&
+                      !any_set({"FDTD_ADJ_GATHER", "FDTD_ADJ_CHUNKS", "FDTD_ADJ_FUSE", "FDTD_INTERIOR"});
     const size_t hist_bytes = (size_t)(Kseg + 1) * 3 * nb * sizeof(float);
     const size_t ck_bytes = state_bytes(c);
     // segmented runs double-buffer the history: with launched reverse sweeps,
