@@ -350,6 +350,14 @@ bool any_set(std::initializer_list<const char *> names)
     return false;
 }
 
+// The fused step's second buffers: the fields and the psi of the E sweep.
+size_t second_bytes(const fdtd_ctx *c)
+{
+    size_t b = 6 * (size_t)c->field_elems * c->esz;
+    for (int p : {0, 1, 4, 5, 8, 9}) b += std::max<size_t>(c->psi_elems[p], 1) * c->esz;
+    return b;
+}
+
 // The fused step's tiling and its second buffers; without the memory for
 // them the context steps with the two sweeps.
 //
@@ -364,7 +372,9 @@ bool any_set(std::initializer_list<const char *> names)
 // 256^3 262 / 277.  Magnetic 512x512x256 1094 / 1081, 640x400x256 1055 / 993;
 // below 512x512x200 900 / 922, 512x512x128 573 / 634, 256^3 280 / 328.
 // FDTD_FUSED=0 / 1 overrides it; a switch that only the sweeps have asks for
-// those.  Blocks of 16 planes, halved until a launch
+// those.  The second buffers take at most an eighth of the memory that is free:
+// what a program allocates next, another context or a tensor, fits as before but
+// for that eighth.  Blocks of 16 planes, halved until a launch
 // has 4096 workgroups (256^3: 8 planes 281 us, 16 planes 296).
 void setup_fused(fdtd_ctx *c)
 {
@@ -382,6 +392,12 @@ void setup_fused(fdtd_ctx *c)
     const double inner = (double)(ib[3] - ib[0]) * tile_cols() * (ib[4] - ib[1]) * by * (ib[5] - ib[2]) * c->kchunk_f;
     const bool uni = c->h_mode == CLS_UNIFORM;
     if (!force && (cells < (uni ? 24e6 : 60e6) || inner < (uni ? 0.375 : 0.5) * cells)) return;
+
+    size_t freeb = 0, totb = 0;
+    if (!force && (hipMemGetInfo(&freeb, &totb) != hipSuccess || second_bytes(c) > freeb / 8)) {
+        (void)hipGetLastError();
+        return;
+    }
 
     const size_t n_allocs = c->allocs.size();
     const uint64_t bytes = c->dev_bytes;
@@ -1366,8 +1382,10 @@ static int adjoint_call(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int
     if (K < 0) {
         // automatic: the design history of the whole run when it fits in half
         // the free device memory (no recompute), else checkpoints every
-        // ceil(sqrt(n)) steps
+        // ceil(sqrt(n)) steps.  (The fused step's second buffers count as free:
+        // they are given back below where the gradient needs them.)
         HIPCHK(c, hipMemGetInfo(&freeb, &totb));
+        if (c->fused) freeb += second_bytes(c);
         const size_t all = (size_t)(n + 1) * 3 * nb * sizeof(float) + adj_bytes + (size_t)std::max(np, 1) * n * 4;
         K = all < freeb / 2 ? 0 : (int)std::ceil(std::sqrt((double)n));
     }
@@ -1509,6 +1527,10 @@ static int adjoint_call(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int
             adj_fuse_tiles(aa, c->built.e_first, c->built.h_first, b.sb, quiet, noisy);
         const size_t pair_bytes = 6 * (size_t)c->field_elems * 4 + (quiet.size() + noisy.size() + 2) * 4;
         if (!quiet.empty()) HIPCHK(c, hipMemGetInfo(&freeb, &totb));
+        if (!quiet.empty() && c->fused && pair_bytes >= freeb / 2 && pair_bytes < (freeb + second_bytes(c)) / 2) {
+            release_fused(c);   // (the reverse pass gains more than the forward step loses)
+            HIPCHK(c, hipMemGetInfo(&freeb, &totb));
+        }
         if (!quiet.empty() && pair_bytes < freeb / 2) {
             for (int q = 0; q < 6; ++q) {
                 char *f = (char *)mem.get((size_t)c->field_elems * 4);
