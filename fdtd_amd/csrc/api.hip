@@ -241,17 +241,14 @@ bool box_in_grid(const fdtd_ctx *c, int i, int j, int k)
     return i >= 0 && j >= 0 && k >= 0 && i < c->in.nx && j < c->in.ny && k < c->in.nz;
 }
 
-// Zero every piece of time-dependent state.
+// Zero every piece of time-dependent state.  (Not the fused step's second
+// buffers, cleared when they are made: a step writes every value of theirs that
+// is ever read, and nothing writes the rest.)
 int zero_state(fdtd_ctx *c)
 {
     for (int f = 0; f < 6; ++f) {
         if (c->fields[f]) HIPCHK(c, hipMemsetAsync(c->fields[f], 0, (size_t)c->field_elems * c->esz, c->stream));
     }
-    for (int f = 0; f < 6; ++f)
-        if (c->fields2[f]) HIPCHK(c, hipMemsetAsync(c->fields2[f], 0, (size_t)c->field_elems * c->esz, c->stream));
-    for (int p = 0; p < 12; ++p)
-        if (c->psi_elems[p] && c->psi2[p])
-            HIPCHK(c, hipMemsetAsync(c->psi2[p], 0, c->psi_elems[p] * c->esz, c->stream));
     for (int q = 0; q < 2; ++q)
         if (c->qarr[q]) HIPCHK(c, hipMemsetAsync(c->qarr[q], 0, c->qarr_bytes, c->stream));
     for (int p = 0; p < 12; ++p)
@@ -406,7 +403,15 @@ void setup_fused(fdtd_ctx *c)
     for (int f = 0; f < 6 && !rc; ++f) rc = dev_alloc(c, &c->fields2[f], (size_t)c->field_elems * c->esz);
     for (int p : {0, 1, 4, 5, 8, 9})
         if (!rc) rc = dev_alloc(c, &c->psi2[p], std::max<size_t>(c->psi_elems[p], 1) * c->esz);
+    for (int f = 0; f < 6 && !rc; ++f)
+        if (hipMemsetAsync(c->fields2[f], 0, (size_t)c->field_elems * c->esz, c->stream) != hipSuccess) rc = FDTD_E_DEVICE;
+    for (int p : {0, 1, 4, 5, 8, 9})
+        if (!rc && c->psi_elems[p] &&
+            hipMemsetAsync(c->psi2[p], 0, c->psi_elems[p] * c->esz, c->stream) != hipSuccess)
+            rc = FDTD_E_DEVICE;
     if (rc) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(c->stream);
         while (c->allocs.size() > n_allocs) {
             (void)hipFree(c->allocs.back());
             c->allocs.pop_back();
