@@ -118,7 +118,7 @@ struct fdtd_ctx {
     int adj_segments = 0;
     uint64_t adj_bytes = 0;         // peak device memory of the last adjoint run
     hipEvent_t adj_ev[3] = {};      // timing events of the adjoint (made at create)
-    float *stage = nullptr;         // pinned memory of fdtd_get_field, two pieces of STAGE floats
+    float *stage = nullptr;         // pinned memory of fdtd_get_field, up to two pieces
     hipEvent_t stage_ev[2] = {};
     unsigned char *scratch = nullptr;   // this device's copy of the static scratch
 };
@@ -1080,8 +1080,6 @@ hipError_t do_step(fdtd_ctx *c, const KArgs &base, int m, hipEvent_t ev0 = nullp
     if (ev3) (void)hipEventRecord(ev3, c->stream);
     return e;
 }
-
-constexpr size_t STAGE = 1 << 20;   // floats of a piece of fdtd_get_field
 
 // The fewest steps that pay for one launch -- the launch itself, loading and
 // storing the tiles, reading its flag -- by the units a wave holds.  us per
@@ -2182,34 +2180,42 @@ int fdtd_get_field(fdtd_ctx *c, int comp, float *out, size_t n)
     const size_t cells = (size_t)nx * ny * nz;
     if (n < cells) return fail(c, FDTD_E_INVALID, "output too small");
     DeviceGuard dg(c->device);
-    // two pieces of pinned memory, made at the first call and kept: the GPU
-    // packs and converts one while the other is copied out.  Through a copy of
-    // the padded array in pageable memory and a loop here, the six fields of
-    // 150x131x118 took 14.5 ms; so 6.3, most of it the copy out (9 GB/s).
+    // two pieces of pinned memory, made at the first call and kept: the GPU packs
+    // and converts one while the other is copied out.  Through a copy of the
+    // padded array in pageable memory and a loop here, the six fields of
+    // 150x131x118 took 14.5 ms; so 6.3, most of it the copy out (9 GB/s).  The
+    // host's first use of the pieces costs 1.7 us for each 4 KB of them, so they
+    // are no larger than the reads after it need: us, a context's first read / six
+    // later ones, pieces of 2^16, 2^17 and 2^20 values: 64^3 350 / 355, 560 / 325,
+    // 535 / 390; 100x96x90 490 / 1050, 670 / 850, 1530 / 1150; 150x131x118 960 / 2860,
+    // 1100 / 2440, 3470 / 2550; 2^17, 2^19, 2^20: 160^3 1390 / 4460, 2500 / 4170, 3810 /
+    // 4150; 256x256x200 3170 / 14900, 3590 / 12000, 5170 / 11500.
+    const size_t piece = cells <= (size_t)1 << 20 ? 1 << 16 : cells <= (size_t)3 << 20 ? 1 << 17 : 1 << 19;
+    const size_t stage = std::min(cells, 2 * piece);
     if (!c->stage) {
         for (auto &e : c->stage_ev)
             if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        if (hipHostMalloc((void **)&c->stage, 2 * STAGE * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc((void **)&c->stage, stage * sizeof(float), hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             c->stage = nullptr;
-            return fail(c, FDTD_E_NOMEM, "pinned host memory (%zu bytes)", 2 * STAGE * sizeof(float));
+            return fail(c, FDTD_E_NOMEM, "pinned host memory (%zu bytes)", stage * sizeof(float));
         }
     }
     const char *base = (const char *)c->fields[comp] + (size_t)c->ka.plane * c->esz;
     const std::uint8_t *qe = c->qexp[comp] ? c->qexp[comp] + (size_t)c->ka.plane / BQ_BLOCK * BQ_STRIDE : nullptr;
     const float un = c->built.probe_unscale[comp];
-    const size_t pieces = (cells + STAGE - 1) / STAGE;
+    const size_t pieces = (cells + piece - 1) / piece;
     for (size_t p = 0; p <= pieces; ++p) {
         if (p < pieces) {
-            const size_t g = p * STAGE, len = std::min(STAGE, cells - g);
-            HIPCHK(c, launch_unpack(c->in.storage, base, qe, c->stage + p % 2 * STAGE, (std::uint32_t)g,
+            const size_t g = p * piece, len = std::min(piece, cells - g);
+            HIPCHK(c, launch_unpack(c->in.storage, base, qe, c->stage + p % 2 * piece, (std::uint32_t)g,
                                     (std::uint32_t)len, nx, px, un, c->stream));
             HIPCHK(c, hipEventRecord(c->stage_ev[p % 2], c->stream));
         }
         if (p > 0) {
-            const size_t g = (p - 1) * STAGE, len = std::min(STAGE, cells - g);
+            const size_t g = (p - 1) * piece, len = std::min(piece, cells - g);
             HIPCHK(c, hipEventSynchronize(c->stage_ev[(p - 1) % 2]));
-            std::memcpy(out + g, c->stage + (p - 1) % 2 * STAGE, len * sizeof(float));
+            std::memcpy(out + g, c->stage + (p - 1) % 2 * piece, len * sizeof(float));
         }
     }
     return FDTD_OK;
