@@ -221,8 +221,11 @@ __device__ __forceinline__ void e_update(const EPlane &p, const Coef &t, const K
     hy_km = carry(hyc);
 }
 
+// (The argument block by value: by reference the compiler keeps more of it in
+// scalar registers across the march and spills them, 2 to 4 % of a step where
+// the general variant runs alone.)
 template <class T, int CM, int V>
-__device__ __forceinline__ void e_tile(const KArgs &a, const int m, const int tx, const int ty, const int tz)
+__device__ __forceinline__ void e_tile(const KArgs a, const int m, const int tx, const int ty, const int tz)
 {
     ECol cc;
     cc.i = tx * TX + (int)(threadIdx.x & (TX - 1));
@@ -467,7 +470,7 @@ __device__ __forceinline__ void h_update(const HPlane &p, const Coef &t, const K
 }
 
 template <class T, int CM, int V>
-__device__ __forceinline__ void h_tile(const KArgs &a, const int m, const int tx, const int ty, const int tz)
+__device__ __forceinline__ void h_tile(const KArgs a, const int m, const int tx, const int ty, const int tz)
 {
     HCol cc;
     cc.i = tx * TX + (int)(threadIdx.x & (TX - 1));

@@ -32,12 +32,17 @@ namespace fdtd {
 // step, a launch each / one launch: 150x131x118 70 / 52, 203x149x97 with
 // magnetic classes 86 / 65, 400x130x70 82 / 67, 320x320x130 magnetic 234 /
 // 226, 512x512x64 322 / 310.
-template <class T, int CM, int ST>
+// GEN: the general variant alone (no interior box, light-cone steps), in a
+// kernel without the others: block-scaled H with one class needs 89 registers
+// for 97, five waves per SIMD for four.  us per step, block-scaled int16, as one of
+// the variants / alone (and a launch for each variant): 140x134x84 51.1 / 48.6
+// (50.1), 264x47x53 27.9 / 26.7 (27.8), 83x62x88 32.3 / 31.2 (32.2).
+template <class T, int CM, int ST, bool GEN>
 __global__ void __launch_bounds__(TX * BY) E_OCC e_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x;
     int tx, ty, tz;
-    if (b < ng) {
+    if (GEN || b < ng) {
         tile_of_region<V_GEN>(a, tx, ty, tz, b);
         e_tile<T, CM, V_GEN | ST>(a, m, tx, ty, tz);
     } else if (b < ng + nx) {
@@ -48,12 +53,12 @@ __global__ void __launch_bounds__(TX * BY) E_OCC e_kernel(const KArgs a, const i
         e_tile<T, CM, V_IN | ST>(a, m, tx, ty, tz);
     }
 }
-template <class T, int CM, int ST>
+template <class T, int CM, int ST, bool GEN>
 __global__ void __launch_bounds__(TX * BY) H_OCC h_kernel(const KArgs a, const int m, const int ng, const int nx)
 {
     const int b = blockIdx.x;
     int tx, ty, tz;
-    if (b < ng) {
+    if (GEN || b < ng) {
         tile_of_region<V_GEN>(a, tx, ty, tz, b);
         h_tile<T, CM, V_GEN | ST>(a, m, tx, ty, tz);
     } else if (b < ng + nx) {
@@ -66,21 +71,27 @@ __global__ void __launch_bounds__(TX * BY) H_OCC h_kernel(const KArgs a, const i
 }
 
 // ---- launchers --------------------------------------------------------------
+template <class T, int ST, bool GEN>
+static void launch_g(bool efield, int mode, const KArgs &a, int m, int ng, int nx, int nb, hipStream_t s)
+{
+    dim3 grid(ng + nx + nb), block(TX * BY);
+    if (efield) {
+        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((e_kernel<T, CLS_UNIFORM, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((e_kernel<T, CLS_U16, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((e_kernel<T, CLS_U32, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+    } else {
+        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((h_kernel<T, CLS_UNIFORM, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+        else if (mode == CLS_U16) hipLaunchKernelGGL((h_kernel<T, CLS_U16, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+        else hipLaunchKernelGGL((h_kernel<T, CLS_U32, ST, GEN>), grid, block, 0, s, a, m, ng, nx);
+    }
+}
 template <class T, int ST>
 static hipError_t launch_t(bool efield, int mode, const KArgs &a, int m, hipStream_t s)
 {
     int nb, nx, nzt, ng;   // nzt = 0: the forward sweeps run without zsplit
     region_tiles(a, nb, nx, nzt, ng);
-    dim3 grid(nb + nx + ng), block(TX * BY);
-    if (efield) {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((e_kernel<T, CLS_UNIFORM, ST>), grid, block, 0, s, a, m, ng, nx);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((e_kernel<T, CLS_U16, ST>), grid, block, 0, s, a, m, ng, nx);
-        else hipLaunchKernelGGL((e_kernel<T, CLS_U32, ST>), grid, block, 0, s, a, m, ng, nx);
-    } else {
-        if (mode == CLS_UNIFORM) hipLaunchKernelGGL((h_kernel<T, CLS_UNIFORM, ST>), grid, block, 0, s, a, m, ng, nx);
-        else if (mode == CLS_U16) hipLaunchKernelGGL((h_kernel<T, CLS_U16, ST>), grid, block, 0, s, a, m, ng, nx);
-        else hipLaunchKernelGGL((h_kernel<T, CLS_U32, ST>), grid, block, 0, s, a, m, ng, nx);
-    }
+    if (nb + nx == 0) launch_g<T, ST, true>(efield, mode, a, m, ng, nx, nb, s);
+    else launch_g<T, ST, false>(efield, mode, a, m, ng, nx, nb, s);
     return hipGetLastError();
 }
 
