@@ -304,9 +304,15 @@ int choose_chunks(const fdtd_ctx *c, int tiles, int planes, const char *planes_e
 // 117 / 93, 250x150x60 38.6 / 36.2, 128x200x200 62 / 55; block-scaled int16
 // 220x220x200 170 / 134, 128x128x100 42.7 / 38.6; with 64 idle columns of 256
 // FP16 180x180x160 66.3 / 67.4, 160x160x150 55 / 59; FP32 112x150x200 74 / 70,
-// 100x80x70 19.9 / 18.2.  FDTD_INTERIOR=0, or a y or z axis without interior
-// tiles, leaves the box empty (z range [0, 0)) and every tile to the general
-// variant.
+// 100x80x70 19.9 / 18.2.  128-cell tiles do so only where half of them lie in
+// those rows and z-blocks, or the z-blocks are long: a pair tile beside two of the
+// general variant's is the longer wait.  By the share of the tiles: block-scaled
+// 212x45x91 (0.31) 29.4 / 31.5, 97x48x83 (0.37) 19.8 / 23.0, 115x54x60 (0.47) 18.8 /
+// 19.4, 73x198x76 (0.53) 45.9 / 43.9, 203x70x160 (0.65) 56.4 / 51.3; of 18 grids
+// below a half 13 were slower so, of 52 others 3 (by 4 % at most); blocks of nine
+// planes: FP16 232x243x74 (0.39) 66.3 / 59.9.  FDTD_INTERIOR=0, or a y or z
+// axis without interior tiles, leaves the box empty (z range [0, 0)) and every
+// tile to the general variant.
 // beyond: cells past the tile's high sides that must lie off the slabs too
 // (the fused step evaluates one).
 void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int beyond = 0)
@@ -320,6 +326,7 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
     const int nts[3] = {(in.nx + tile_cols - 1) / tile_cols, (in.ny + by - 1) / by, (in.nz + kchunk - 1) / kchunk};
     const int w[3] = {tile_cols, by, kchunk}, nn[3] = {in.nx, in.ny, in.nz};
     int box[6];
+    bool edge_only = false;
     for (int ax = 0; ax < 3; ++ax) {
         const int lo_cells = std::max(L[2 * ax], 1), hi_cells = nn[ax] - std::max(L[2 * ax + 1], 1);
         int lo = nts[ax], hi = 0;
@@ -332,10 +339,14 @@ void sweep_split(fdtd_ctx *c, int sweep, int tile_cols, int by, int kchunk, int 
             const int t64 = (in.nx + 63) / 64;
             if (ax > 0 || sweep == 2 || (tile_cols > 64 && t64 % 2 != 0 && t64 < 5)) return;
             lo = hi = 0;
+            edge_only = true;
         }
         box[ax] = lo;
         box[ax + 3] = hi;
     }
+    if (edge_only && tile_cols > 64 && kchunk < 8 &&
+        2L * (box[4] - box[1]) * (box[5] - box[2]) < (long)nts[1] * nts[2])
+        return;
     for (int q = 0; q < 6; ++q) ib[q] = box[q];
 }
 
