@@ -4,7 +4,7 @@
 // in one launch: the same tiles, one per CU, and the same exchange of rows
 // between them (the transposed H quantities of the high sides before the E
 // half-step, the transposed E quantities of the low sides before the H one).
-// Launched one by one, a reverse step of 128x128x64 takes 47 us however its
+// Launched one by one, a reverse step of 128x128x64 takes 44 us however its
 // blocks are cut: launches, and 24 arrays read or written through chains
 // of dependent trips to memory.
 //
@@ -19,8 +19,8 @@
 //
 // What bounds it: as in persist.hip, the exchange and then the vector
 // instructions of a half-step at four waves per SIMD.  Reverse step of
-// 128x128x64 (four units a wave) 47.0 us launched, 21.1 in one launch; of 64^3
-// (one) 18.4, 5.9; of 96^3 (five, which spill 27 registers) 43.6, 26.8.
+// 128x128x64 (four units a wave) 44.0 us launched, 21.1 in one launch; of 64^3
+// (one) 18.4, 6.0; of 96^3 (five, which spill 27 registers) 43.2, 26.5.
 //
 // The arithmetic of a cell is that of adjoint.hip (adj_e_kernel,
 // adj_h_kernel), in the same order; the results are the same bits.

@@ -4,9 +4,9 @@
 // (fdtdrav.h:3425-4387), and its per-step driver, solver (fdtdrav.h:3188-3422),
 // for one device: the z-slab split and ghost-plane copies of the reference
 // collapse into a single domain whose neighbour planes are plain HBM reads.
-// All work goes to one non-blocking stream; a step is the E sweep then the
-// H sweep (one launch per non-empty region variant each), with no host
-// synchronisation between them.
+// All work goes to one non-blocking stream, with no host synchronisation
+// between steps: a step is the E sweep then the H sweep, a launch each; one pass
+// over large FP32 grids; and small grids run many steps in one launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -458,9 +458,9 @@ void release_fused(fdtd_ctx *c)
 // forward units.  Rule: wherever the forward steps run in one launch and a
 // tile's units and events fit 160 KB of LDS (76 units; any storage form: the
 // reverse state is FP32).  All of it is faster that way; a reverse step, us,
-// launched / in one launch: 28x24x22 14.3 / 5.3, 64^3 18.4 / 5.9, 127x100x50
-// 32.6 / 14.0, 300x60x40 54.0 / 17.1, 128x128x64 47.0 / 21.1, 112x96x90 46.1 /
-// 28.0, 96^3 43.6 / 26.8.  FDTD_ADJ_PERSIST=0 turns it off.
+// launched / in one launch: 28x24x22 13.4 / 5.4, 64^3 18.4 / 6.0, 127x100x50 30.8 /
+// 13.3, 300x60x40 34.8 / 17.0, 128x128x64 44.0 / 21.1, 112x96x90 43.1 / 26.7, 96^3
+// 43.2 / 26.5.  FDTD_ADJ_PERSIST=0 turns it off.
 void setup_radj(fdtd_ctx *c, const std::vector<PTile> &ptiles, const std::vector<PUnit> (&units)[2], int gy, int tz)
 {
     const SceneIn &in = c->in;
@@ -650,9 +650,9 @@ hipError_t launch_steps(fdtd_ctx *c, const KArgs &a)
 // The rule: FP32, FP16 or BF16 storage, one H class, and a tiling of at most
 // 256 tiles of 80 row segments (about 1.3 M cells), each with at most
 // P_MAX_EVENTS source edges and probes.  Every such grid measured is faster in
-// one launch, us per step, sweeps / one launch of 300 steps: 64^3 13.5 / 3.9,
-// 300x60x40 34.7 / 11.3, 110x150x53 27.1 / 15.2, 128x128x64 27.8 / 14.6 (FP16
-// 23.0 / 16.7), 128x128x80 32.8 / 17.1, 12x9x8 10.0 / 3.2; and from 6 to 10 steps
+// one launch, us per step, sweeps / one launch of 300 steps: 64^3 12.2 / 3.9,
+// 300x60x40 18.0 / 11.4, 110x150x53 22.0 / 14.6, 128x128x64 19.4 / 14.5 (FP16 22.4 /
+// 16.5), 128x128x80 22.9 / 17.2, 96^3 19.6 / 14.1, 12x9x8 8.0 / 3.0; and from 6 to 10 steps
 // on (persist_min_steps).  FDTD_PERSIST=0 turns it off, and so does a switch of
 // the launched sweeps, which asks for those.
 void setup_persist(fdtd_ctx *c)

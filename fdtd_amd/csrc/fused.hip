@@ -47,7 +47,7 @@ namespace fdtd {
 
 typedef std::uint32_t u32;
 
-constexpr int FY = 7;   // rows of a tile; the eighth wave evaluates the edge cells   // rows of a tile; the eighth wave evaluates the edge cells
+constexpr int FY = 7;   // rows of a tile; the eighth wave evaluates the edge cells
 
 // One column of cells (i, j): predicates, slab indices, CPML profiles.
 struct FCol {

@@ -841,7 +841,8 @@ static void launch_pair_all(bool efield, int mode, const KArgs &a, int m, int ng
 }
 
 // One half-step.  a.tiles_x counts 128-cell tile columns.  gen_cells: the
-// general variant runs as the one-cell kernel.
+// general variant runs as the one-cell kernel; without it (a switch) the own
+// values always go past the caches.
 template <class T>
 hipError_t launch_pair_t(bool efield, int mode, const KArgs &a, int m, hipStream_t s, bool gen_cells)
 {

@@ -20,8 +20,9 @@
 // What bounds it: the exchange (two trips through memory and two barriers a
 // step, 3.2 us where a tile is one row) and, per unit, the vector
 // instructions of a half-step at four waves per SIMD (about 1.5 us for each
-// unit a wave holds).  64^3 (one unit a wave): 12.2 us a step launched, 4.0
-// in one launch; 128x128x64 (four) 27.8 -> 14.6.  Units described by scalar
+// unit a wave holds).  64^3 (one unit a wave): 12.2 us a step launched, 3.9
+// in one launch; 128x128x64 (four) 19.4 -> 14.5 (27.8 with a launch for each
+// region variant).  Units described by scalar
 // loads, coefficients and psi read each step: 64^3 5.4, 128x128x64 20.1 (a
 // wait for any load also waits for the psi and row stores before it, so
 // what can be is kept in registers).

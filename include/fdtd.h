@@ -129,8 +129,11 @@ typedef struct {
     int      storage;            /* FDTD_STORE_*                               */
     double   dt;
     double   last_run_ms;        /* hipEvent time of the last fdtd_run() loop  */
-    double   e_kernel_ms;        /* mean E-kernel launch time (fdtd_profile);
-                                    the whole step's where one pass does both */
+    double   e_kernel_ms;        /* mean E-kernel launch time (fdtd_profile,
+                                    which launches every step by itself, also
+                                    where fdtd_run has many steps in one
+                                    launch); the whole step's where one pass
+                                    does both                                 */
     double   h_kernel_ms;        /* mean H-kernel launch time (fdtd_profile)   */
     double   step_kernel_ms;     /* mean time of one step's launches            */
     int      interior_split;     /* 1: the sweeps run interior / x-edge /
@@ -256,7 +259,11 @@ int fdtd_finalize(fdtd_ctx *ctx, int n_steps);
 
 /* Advance nsteps steps (E then H each step, fdtdrav.h:3188-3422 and the
  * loop of fdtdrav.h:4320-4355).  Blocking; returns FDTD_E_NONFINITE if a
- * probe went non-finite. */
+ * probe went non-finite.  Small grids run many steps in one launch whose
+ * workgroups wait for each other; should one wait for seconds (the GPU held
+ * by other work), the call returns FDTD_E_DEVICE and run, outputs and
+ * checkpoint saves return FDTD_E_STATE until fdtd_reset or
+ * fdtd_checkpoint_restore. */
 int fdtd_run(fdtd_ctx *ctx, int nsteps);
 
 /* Advance one step: the E sweep then the H sweep of step steps_done.
@@ -269,7 +276,9 @@ int fdtd_step(fdtd_ctx *ctx);
 int fdtd_reset(fdtd_ctx *ctx);
 
 /* Run nsteps steps with a HIP event pair around every E and every H launch
- * and store the mean launch times in fdtd_info.  Same results as fdtd_run. */
+ * and store the mean launch times in fdtd_info.  Same results as fdtd_run,
+ * but every step is launched by itself, also on small grids where fdtd_run
+ * has many in one launch. */
 int fdtd_profile(fdtd_ctx *ctx, int nsteps);
 
 int fdtd_get_info(const fdtd_ctx *ctx, fdtd_info *info);
