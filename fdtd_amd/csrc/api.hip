@@ -371,14 +371,17 @@ size_t second_bytes(const fdtd_ctx *c)
 //
 // The rule: FP32 grids of 24 M cells or more (60 M where the H coefficients
 // differ by cell, which costs the fused kernel 16 registers) whose interior
-// tiles hold 3/8 of the cells (half).  The fused pass gains on interior tiles
+// tiles hold 3/8 of the cells (3/5).  The fused pass gains on interior tiles
 // and where the fields are read from HBM; its general variant, with both
 // half-steps' slab state, does not, and its workgroups are fewer and longer.
 // Measured, us per step, sweeps / fused: 512x512x256 1061 / 937, 384x384x200
 // 488 / 446, 448x256x256 468 / 430, 300^3 463 / 448; below the line 288^3 400
 // / 409, 512x300x150 380 / 363, 260x260x300 376 / 398, 320x320x160 254 / 271,
-// 256^3 262 / 277.  Magnetic 512x512x256 1094 / 1081, 640x400x256 1055 / 993;
-// below 512x512x200 900 / 922, 512x512x128 573 / 634, 256^3 280 / 328.
+// 256^3 262 / 277.  Magnetic, by the share of the interior: 512x512x240 (0.61) 1092
+// / 988, 900x300x250 (0.65) 1116 / 1102, 400^3 (0.68) 1110 / 1061, but 1000x260x250
+// (0.66) 1060 / 1088; below the line 512x512x256 (0.56) 1093 / 1102, 900x300x250
+// with a thicker CPML (0.55) 1244 / 1268, 640x400x256 (0.54) 1144 / 1143, 400^3 (0.46)
+// 1185 / 1227; below 60 M 512x512x200 900 / 922, 512x512x128 573 / 634.
 // FDTD_FUSED=0 / 1 overrides it; a switch that only the sweeps have asks for
 // those.  The second buffers take at most an eighth of the memory that is free:
 // what a program allocates next, another context or a tensor, fits as before but
@@ -399,7 +402,7 @@ void setup_fused(fdtd_ctx *c)
     const double cells = (double)in.nx * in.ny * in.nz;
     const double inner = (double)(ib[3] - ib[0]) * tile_cols() * (ib[4] - ib[1]) * by * (ib[5] - ib[2]) * c->kchunk_f;
     const bool uni = c->h_mode == CLS_UNIFORM;
-    if (!force && (cells < (uni ? 24e6 : 60e6) || inner < (uni ? 0.375 : 0.5) * cells)) return;
+    if (!force && (cells < (uni ? 24e6 : 60e6) || inner < (uni ? 0.375 : 0.6) * cells)) return;
 
     size_t freeb = 0, totb = 0;
     if (!force && (hipMemGetInfo(&freeb, &totb) != hipSuccess || second_bytes(c) > freeb / 8)) {
@@ -1542,7 +1545,7 @@ static int adjoint_call(fdtd_ctx *c, const fdtd_objective *obj, int n_steps, int
         const size_t pair_bytes = 6 * (size_t)c->field_elems * 4 + (quiet.size() + noisy.size() + 2) * 4;
         if (!quiet.empty()) HIPCHK(c, hipMemGetInfo(&freeb, &totb));
         if (!quiet.empty() && c->fused && pair_bytes >= freeb / 2 && pair_bytes < (freeb + second_bytes(c)) / 2) {
-            release_fused(c);   // (the reverse pass gains more than the forward step loses)
+            release_fused(c);   // (the same choice as without them)
             HIPCHK(c, hipMemGetInfo(&freeb, &totb));
         }
         if (!quiet.empty() && pair_bytes < freeb / 2) {
